@@ -1,0 +1,94 @@
+// Large-batch GEMM launchers (kernels in bgemm_kernels.h).
+#include "launch.h"
+#include "bgemm_kernels.h"
+
+namespace fl {
+
+namespace {
+
+template <int FMT, int TT, int NW>
+hipError_t launch_one(hipStream_t st, const BgArgs &a) {
+    constexpr size_t lds = (size_t)2 * TT * kPackRec + (FMT == F_Q4K ? NW * 32 * 4 : 0);
+    const auto kern = k_bgemm<FMT, TT, NW>;
+    static const hipError_t attr =
+        hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (attr != hipSuccess) return attr;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(a.nrt * a.ntt * a.ksplit)), dim3(NW * 64), lds, st, a);
+    return hipGetLastError();
+}
+
+template <int FMT, int NW>
+hipError_t launch_tt(int tt, hipStream_t st, const BgArgs &a) {
+    switch (tt) {
+    case 1: return launch_one<FMT, 1, NW>(st, a);
+    case 2: return launch_one<FMT, 2, NW>(st, a);
+    case 3: return launch_one<FMT, 3, NW>(st, a);
+    case 4: return launch_one<FMT, 4, NW>(st, a);
+    }
+    return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+// The plan of least estimated time.  A workgroup of 8 waves (or two of 4
+// waves with at most 2 token tiles) fills a CU; measured per 256-value step
+// and round of the chip on MI355X (28672 x 4096 Q4_K, 2048 tokens): 2.9, 4.3,
+// 5.4 and 7.0 us with 1, 2, 3 and 4 token tiles.  K is split where tiles alone
+// leave CUs idle; the split's partial sums cost a write, a read (4 TB/s
+// together) and a launch.
+BgPlan bgemm_plan(int rows, int cols, int M) {
+    static const double step_us[5] = {0, 2.9, 4.3, 5.4, 7.0};
+    const int tiles = (M + kPackTile - 1) / kPackTile, nst = (cols + 255) / 256;
+    BgPlan best{};
+    double best_us = 0;
+    for (int tt = 1; tt <= std::min(4, tiles); tt++)
+        for (int nw = 8; nw >= (tt <= 2 ? 4 : 8); nw /= 2)
+            for (int want = 1; want <= std::min(nst, kBgMaxSplit); want++) {
+                BgPlan p;
+                p.tt = tt;
+                p.nw = nw;
+                p.ntt = (tiles + tt - 1) / tt;
+                p.nrt = (rows + 32 * nw - 1) / (32 * nw);
+                p.chunk = (nst + want - 1) / want;
+                p.ksplit = (nst + p.chunk - 1) / p.chunk;
+                if (p.ksplit != want) continue;
+                const long long wgs = (long long)p.nrt * p.ntt * p.ksplit, slots = nw == 8 ? 256 : 512;
+                double us = (double)((wgs + slots - 1) / slots) * p.chunk * step_us[tt];
+                if (p.ksplit > 1) us += 4.0 + 2.0 * p.ksplit * M * (double)rows * 4 / 4e6;
+                if (!best.tt || us < best_us) {
+                    best = p;
+                    best_us = us;
+                }
+            }
+    return best;
+}
+
+hipError_t launch_bgemm(int fmt, hipStream_t st, const WDesc &W, const char *xp, int M, const BgPlan &p, float *part) {
+    if (M < 1 || W.rows < 1 || W.cols % 32 || (fmt == F_Q4K && W.cols % 256)) return hipErrorInvalidValue;
+    BgArgs a{};
+    a.W = W;
+    a.xp = xp;
+    a.M = M;
+    a.nst = (W.cols + 255) / 256;
+    a.ksplit = p.ksplit;
+    a.chunk = p.chunk;
+    a.part = part;
+    a.nrt = p.nrt;
+    a.ntt = p.ntt;
+    // every row, token and step belongs to a workgroup, every split has steps
+    if ((long long)p.nrt * p.nw * 32 < W.rows || (long long)p.ntt * p.tt * kPackTile < M ||
+        (long long)p.ksplit * p.chunk < a.nst || (long long)(p.ksplit - 1) * p.chunk >= a.nst)
+        return hipErrorInvalidValue;
+    if (fmt == F_Q4K) return p.nw == 8 ? launch_tt<F_Q4K, 8>(p.tt, st, a) : launch_tt<F_Q4K, 4>(p.tt, st, a);
+    if (fmt == F_Q8_0) return p.nw == 8 ? launch_tt<F_Q8_0, 8>(p.tt, st, a) : launch_tt<F_Q8_0, 4>(p.tt, st, a);
+    return hipErrorNotSupported;
+}
+
+hipError_t launch_quant_pack(hipStream_t st, const float *x, int M, int K, char *xp) {
+    if (M < 1 || K < 32 || K % 32) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_quant_pack, dim3((M + kPackTile - 1) / kPackTile, (K / 32 + 3) / 4), dim3(256), 0, st, x, M, K,
+                       (K + 255) / 256, xp);
+    return hipGetLastError();
+}
+
+}  // namespace fl

@@ -250,6 +250,8 @@ struct fl_ctx {
     size_t part_cap = 0;
     int *d_counters = nullptr;    // [kCounterWords]: split arrivals [0, 1024), fused-launch counts and flag after
     unsigned long long *d_slot = nullptr;
+    char *ws = nullptr;           // workspace of the batched ops (grown to the largest call, see ws_ensure)
+    size_t ws_bytes = 0;
     // model
     bool have_cfg = false, have_weights = false;
     fl_model_config cfg{};
@@ -317,6 +319,7 @@ struct fl_ctx {
 };
 
 constexpr int kVerifyMaxKsplit = 16;
+constexpr int kBatchRows = 2048;  // rows per GEMM of fl_op_batched_dequant_matmul (bounds its workspace)
 constexpr int kVerifyCounters = 4096;  // workgroup columns of a fused verify GEMM
 
 // K-split partials of fl_op_batched_matvec_q8in_noalloc: a file-scope device
@@ -650,6 +653,25 @@ static int ensure_part(fl_ctx *ctx, size_t floats) {
     return 0;
 }
 
+// The batched ops' workspace: activations and partial sums of one call.  Kept
+// with the context (a hipMalloc / hipFree pair per call costs more than the
+// smaller GEMMs) and grown when a call needs more; the ops bound what a call
+// needs by walking large batches in pieces.  The ops enqueue on the context
+// stream only, so a call that follows another cannot overwrite it early; a
+// grown buffer is freed after that stream has drained.
+static int ws_ensure(fl_ctx *ctx, size_t bytes) {
+    if (ctx->ws_bytes >= bytes) return 0;
+    if (ctx->ws) {
+        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+        (void)hipFree(ctx->ws);
+    }
+    ctx->ws = nullptr;
+    ctx->ws_bytes = 0;
+    ALLOC(ctx, ctx->ws, bytes);
+    ctx->ws_bytes = bytes;
+    return 0;
+}
+
 // =====================================================================
 // C-ABI
 // =====================================================================
@@ -756,7 +778,7 @@ void fl_ctx_destroy(fl_ctx *ctx) {
     model_release(ctx);
     void *ptrs[] = {ctx->d_pos, ctx->d_rope_row, ctx->d_part, ctx->d_counters, ctx->d_slot,
                     ctx->sp, ctx->scounts, ctx->sprev, ctx->sstate, ctx->svals, ctx->ssvals, ctx->skeys,
-                    ctx->sskeys, ctx->ssort};
+                    ctx->sskeys, ctx->ssort, ctx->ws};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -1981,8 +2003,9 @@ int fl_op_batched_matvec_q8in(fl_ctx *ctx, const fl_weight *w, int n_tokens, con
     int chunk = 0;
     const int ks = verify_split(*w, n_tokens, chunk);
     const size_t need = (size_t)ks * n_tokens * w->rows;
-    float *part = nullptr;
-    ALLOC(ctx, part, need * 4);
+    const int rc = ws_ensure(ctx, need * 4);
+    if (rc) return rc;
+    float *part = (float *)ctx->ws;
     VgArgs a{};
     a.W = w->desc();
     a.xq = q;
@@ -1995,7 +2018,6 @@ int fl_op_batched_matvec_q8in(fl_ctx *ctx, const fl_weight *w, int n_tokens, con
     hipError_t e = launch_vgemm(w->format, ctx->stream, a);
     if (e == hipSuccess) e = launch_v_store(ctx->stream, part, ks, n_tokens, w->rows, out);
     const hipError_t e2 = hipStreamSynchronize(ctx->stream);
-    (void)hipFree(part);
     HIPCHK(ctx, e);
     HIPCHK(ctx, e2);
     return 0;
@@ -2065,32 +2087,51 @@ int fl_op_batched_dequant_matmul(fl_ctx *ctx, const fl_weight *w, const float *i
     if (batch < 1) return fail(ctx, FL_E_INVALID, "batch %d", batch);
     if (w->format != FL_Q8_0 && w->format != FL_Q4K)
         return fail(ctx, FL_E_UNSUPPORTED, "batched_dequant_matmul for format %d (Q8_0 / Q4_K)", w->format);
-    // quantize_input_q8_0_into of every input row (rows are contiguous and
-    // cols % 32 == 0, so the blocks of all rows are one array)
-    const size_t cols = (size_t)w->cols, nblk = (size_t)batch * cols / 32;
-    int8_t *q = nullptr;
-    float *sc = nullptr;
-    int *sum = nullptr;
-    int rc = dev_alloc(ctx, (void **)&q, (size_t)batch * cols);
-    if (!rc) rc = dev_alloc(ctx, (void **)&sc, nblk * 4);
-    if (!rc) rc = dev_alloc(ctx, (void **)&sum, nblk * 4);
-    if (!rc) {
-        hipLaunchKernelGGL(k_quantize, dim3((unsigned)((nblk + kThreads - 1) / kThreads)), dim3(kThreads), 0,
-                           ctx->stream, input, (int)nblk, q, sc, sum);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) rc = fail(ctx, FL_E_HIP, "quantize: %s", hipGetErrorString(e));
+    const int cols = w->cols;
+    const size_t nblk = (size_t)cols / 32;
+    hipError_t e = hipSuccess;
+    if (batch > kVerifyMaxTokens) {
+        // quantize_input_q8_0_into of every row into the GEMM's packed form,
+        // then one GEMM per kBatchRows rows
+        for (int b0 = 0; b0 < batch && e == hipSuccess; b0 += kBatchRows) {
+            const int n = std::min(kBatchRows, batch - b0);
+            const BgPlan p = bgemm_plan(w->rows, cols, n);
+            const size_t xb = pack_bytes(n, cols);
+            const int rc = ws_ensure(ctx, xb + (p.ksplit > 1 ? (size_t)p.ksplit * n * w->rows * 4 : 0));
+            if (rc) return rc;
+            float *o = out + (size_t)b0 * w->rows, *part = p.ksplit > 1 ? (float *)(ctx->ws + xb) : o;
+            e = launch_quant_pack(ctx->stream, input + (size_t)b0 * cols, n, cols, ctx->ws);
+            if (e == hipSuccess) e = launch_bgemm(w->format, ctx->stream, w->desc(), ctx->ws, n, p, part);
+            if (e == hipSuccess && p.ksplit > 1) e = launch_v_store(ctx->stream, part, p.ksplit, n, w->rows, o);
+        }
+    } else {
+        // quantized rows, then the 16-token GEMM
+        VgArgs a{};
+        a.ksplit = verify_split(*w, batch, a.chunk);
+        auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
+        const size_t qb = up((size_t)batch * cols), sb = up(batch * nblk * 4);
+        const int rc = ws_ensure(ctx, qb + 2 * sb + (size_t)a.ksplit * batch * w->rows * 4);
+        if (rc) return rc;
+        int8_t *q = (int8_t *)ctx->ws;
+        float *sc = (float *)(ctx->ws + qb);
+        int *sum = (int *)(ctx->ws + qb + sb);
+        a.W = w->desc();
+        a.xq = q;
+        a.xs = sc;
+        a.xsum = sum;
+        a.M = batch;
+        a.part = (float *)(ctx->ws + qb + 2 * sb);
+        const size_t nb = batch * nblk;
+        hipLaunchKernelGGL(k_quantize, dim3((unsigned)((nb + kThreads - 1) / kThreads)), dim3(kThreads), 0, ctx->stream,
+                           input, (int)nb, q, sc, sum);
+        e = hipGetLastError();
+        if (e == hipSuccess) e = launch_vgemm(w->format, ctx->stream, a);
+        if (e == hipSuccess) e = launch_v_store(ctx->stream, a.part, a.ksplit, batch, w->rows, out);
     }
-    // then the per-row quantized matvec, kVerifyMaxTokens rows per GEMM
-    for (int b0 = 0; !rc && b0 < batch; b0 += kVerifyMaxTokens) {
-        const int n = std::min(kVerifyMaxTokens, batch - b0);
-        rc = fl_op_batched_matvec_q8in(ctx, w, n, q + (size_t)b0 * cols, sc + (size_t)b0 * (cols / 32),
-                                       sum + (size_t)b0 * (cols / 32), out + (size_t)b0 * w->rows);
-    }
-    (void)hipStreamSynchronize(ctx->stream);
-    if (q) (void)hipFree(q);
-    if (sc) (void)hipFree(sc);
-    if (sum) (void)hipFree(sum);
-    return rc;
+    const hipError_t e2 = hipStreamSynchronize(ctx->stream);
+    HIPCHK(ctx, e);
+    HIPCHK(ctx, e2);
+    return 0;
 }
 
 int fl_op_prefill_attention(fl_ctx *ctx, const float *q, const float *k, const float *v, int seq_len, int num_heads,

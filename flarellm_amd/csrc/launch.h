@@ -10,6 +10,7 @@
 #include <utility>
 
 #include "attn_kernels.h"
+#include "bgemm_args.h"
 #include "mvs_kernels.h"
 #include "verify_args.h"
 
@@ -170,6 +171,16 @@ hipError_t launch_out_seq(int fmt, hipStream_t st, const WDesc &W, const float *
 // MFMA output projection with f32 input for up to 8 tokens (mvo.hip)
 struct MvoArgs;
 hipError_t launch_mvo(int fmt, hipStream_t st, const MvoArgs &a);
+
+// large-batch GEMM (bgemm.hip): workgroup tiles of 32 nw rows x 32 tt tokens,
+// K in ksplit chunks of 256-value steps
+constexpr int kBgMaxSplit = 32;
+struct BgPlan {
+    int tt, nw, nrt, ntt, ksplit, chunk;
+};
+BgPlan bgemm_plan(int rows, int cols, int M);
+hipError_t launch_bgemm(int fmt, hipStream_t st, const WDesc &W, const char *xp, int M, const BgPlan &p, float *part);
+hipError_t launch_quant_pack(hipStream_t st, const float *x, int M, int K, char *xp);
 
 // speculative verify (verify.hip)
 hipError_t launch_vgemm(int fmt, hipStream_t st, const VgArgs &a);
