@@ -28,9 +28,9 @@ HIP_FLAGS = [
 CXX_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-fopenmp", "-ffp-contract=off"]
 
 
-# Per-source flags.  verify.hip, bgemm.hip: MFMA results in VGPRs (no
-# accumulator-register copies before the fp32 block terms of the GEMMs).
-SOURCE_FLAGS = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for f in ("verify.hip", "bgemm.hip")}
+# Per-source flags.  verify.hip, bgemm.hip, attw.hip: MFMA results in VGPRs (no
+# accumulator-register copies before the fp32 block terms or the softmax).
+SOURCE_FLAGS = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for f in ("verify.hip", "bgemm.hip", "attw.hip")}
 
 
 def _run(cmd: list[str]) -> None:
@@ -39,7 +39,7 @@ def _run(cmd: list[str]) -> None:
 
 
 HIP_SOURCES = ["flare_hip.hip", "mvs_q8_0.hip", "mvs_q4k.hip", "mvs_f32.hip", "attn.hip", "verify.hip", "mvo.hip", "seq.hip",
-               "sample.hip", "fused.hip", "bgemm.hip"]
+               "sample.hip", "fused.hip", "bgemm.hip", "attw.hip"]
 HOST_SOURCES = ["synth.cpp", "generate.cpp", "gguf.cpp"]
 
 

@@ -91,4 +91,30 @@ hipError_t launch_quant_pack(hipStream_t st, const float *x, int M, int K, char 
     return hipGetLastError();
 }
 
+// workgroups of kernels that map them with pack_wg: tiles in groups of 8
+static unsigned pack_grid(int M, int nchunk) {
+    return (unsigned)((M + 8 * kPackTile - 1) / (8 * kPackTile) * 8 * kPackTile * nchunk);
+}
+
+hipError_t launch_b_resnorm(int pro, hipStream_t st, const float *part, int ksplit, int M, int H, float *x,
+                            const float *w, float eps, char *xp) {
+    if (H % 32 || H > kResnormMaxH || M < 1) return hipErrorInvalidValue;
+    const auto kern = pro == PRO_NORMQ0 ? k_b_resnorm<PRO_NORMQ0> : k_b_resnorm<PRO_NORMQ1>;
+    hipLaunchKernelGGL(kern, dim3(pack_grid(M, 1)), dim3(kResnormThreads), 0, st, part, ksplit, M, H, x, w, eps,
+                       (H + 255) / 256, xp);
+    return hipGetLastError();
+}
+
+hipError_t launch_b_residual_row(hipStream_t st, const float *part, int ksplit, size_t plane, int H, float *x) {
+    hipLaunchKernelGGL(k_b_residual_row, dim3((H + 255) / 256), dim3(256), 0, st, part, ksplit, plane, H, x);
+    return hipGetLastError();
+}
+
+hipError_t launch_b_silu(hipStream_t st, const float *part, int ksplit, int M, int F, char *xp) {
+    if (F % 32 || M < 1) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_b_silu, dim3(pack_grid(M, (F + 1023) / 1024)), dim3(256), 0, st, part, ksplit, M, F,
+                       (F + 255) / 256, xp);
+    return hipGetLastError();
+}
+
 }  // namespace fl

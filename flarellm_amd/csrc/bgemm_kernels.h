@@ -12,22 +12,10 @@
 // result, so that scale is one register).
 #pragma once
 
-#include "bgemm_args.h"
+#include "bgemm_pack.h"
+#include "verify_args.h"
 
 namespace fl {
-
-typedef _Float16 h8x_t __attribute__((ext_vector_type(8)));
-typedef _Float16 h2x_t __attribute__((ext_vector_type(2)));
-typedef __bf16 b8x_t __attribute__((ext_vector_type(8)));
-typedef float f16x_t __attribute__((ext_vector_type(16)));
-typedef float f32x_t __attribute__((ext_vector_type(32)));
-typedef uint32_t u4x_t __attribute__((ext_vector_type(4)));
-
-// 16 bytes per lane from memory to LDS at lds + 16 * lane (lds wave-uniform)
-__device__ __forceinline__ void copy_to_lds(const char *g, char *lds) {
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)g,
-                                     (__attribute__((address_space(3))) void *)lds, 16, 0, 0);
-}
 
 __device__ __forceinline__ h8x_t as_h8(u4x_t v) { return __builtin_bit_cast(h8x_t, v); }
 __device__ __forceinline__ uint32_t h2_bits(h2x_t v) { return __builtin_bit_cast(uint32_t, v); }
@@ -62,28 +50,6 @@ __device__ __forceinline__ void i8_pairs(uint32_t w0, uint32_t w1, uint32_t (&o)
                            __builtin_amdgcn_perm(0x64646464u, b, 0x04030401u)};
 #pragma unroll
     for (int i = 0; i < 4; i++) o[i] = h2_bits(bits_h2(v[i]) - bias);
-}
-
-// Where a token's value k of a packed row lies in its tile's record (bytes;
-// k within a step): the inverse of the layout above.
-__device__ __forceinline__ int pack_off(int t, int k) {
-    // within 8 values: order 0 2 1 3 4 6 5 7 is its own inverse
-    const int e = (k & 4) | ((k & 1) << 1) | ((k >> 1) & 1);
-    return (k >> 5) * 2048 + ((k >> 3) & 1) * 1024 + ((t & 31) + 32 * ((k >> 4) & 1)) * 16 + e * 2;
-}
-
-// A block's scale and s * sum q in a record (blk within the step).
-__device__ __forceinline__ void pack_scale(char *rec, int t, int blk, float s, int sum) {
-    *(float *)(rec + kPackScale + blk * 128 + (t & 31) * 4) = s;
-    // three bfloat16 parts, each the truncated rest of the one before: 24 bits
-    float v = s * (float)sum;
-    uint16_t *m = (uint16_t *)(rec + kPackMin) + (t & 31) * 8 + blk;
-#pragma unroll
-    for (int p = 0; p < 3; p++) {
-        const uint32_t b = __float_as_uint(v) & 0xFFFF0000u;
-        m[p * 256] = (uint16_t)(b >> 16);
-        v -= __uint_as_float(b);
-    }
 }
 
 // quantize_input_q8_0_into (model.rs:5534-5571) of M f32 rows into packed
@@ -121,6 +87,113 @@ __global__ __launch_bounds__(256) void k_quant_pack(const float *x, int M, int K
     *(h8x_t *)o = c[0];
     *(h8x_t *)(o + 1024) = c[1];
     if (h == 0) pack_scale(rec, l31, blk & 7, d, sum);
+}
+
+// Workgroup -> (token, chunk): the 32 tokens of a tile share a record, so they
+// run on one XCD (blockIdx % 8) in a row and its L2 merges their 8-byte pieces.
+__device__ __forceinline__ void pack_wg(int nchunk, int &t, int &chunk) {
+    const int i = blockIdx.x >> 3;
+    chunk = (i >> 5) % nchunk;
+    t = (((i >> 5) / nchunk) * 8 + (blockIdx.x & 7)) * kPackTile + (i & 31);
+}
+
+// The Q8_0 block of 32 values held 4 a thread by 8 neighbouring threads, into a
+// record (quantize_input_q8_0_into arithmetic); k = the first value's index
+// within the step.
+__device__ __forceinline__ void pack_block8(const float (&y)[4], bool in, char *rec, int t, int k) {
+    float amax = fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), fmaxf(fabsf(y[2]), fabsf(y[3])));
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+    const float d = amax / 127.0f;
+    const float id = (d != 0.0f) ? 127.0f / amax : 0.0f;
+    int q[4], sum = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        q[j] = q8_code(y[j] * id);
+        sum += q[j];
+    }
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) sum += __shfl_xor(sum, o, 64);
+    if (!in) return;
+    pack_codes4(rec, t, k, q[0], q[1], q[2], q[3]);
+    if ((k & 31) == 0) pack_scale(rec, t, k >> 5, d, sum);
+}
+
+__device__ __forceinline__ v4f_t part_sum4(const float *part, int ksplit, size_t plane, size_t at) {
+    v4f_t v = *(const v4f_t *)(part + at);
+    for (int k = 1; k < ksplit; k++) v += *(const v4f_t *)(part + k * plane + at);
+    return v;
+}
+
+// Residual add, RMSNorm and Q8_0 quantization of M tokens as k_v_resnorm
+// (rmsnorm_quantize_q8_0 / rmsnorm_into + quantize, model.rs:5581-5640 /
+// 7456-7477), the codes into packed records.  One workgroup per token.
+template <int PRO>
+__global__ __launch_bounds__(kResnormThreads) void k_b_resnorm(const float *part, int ksplit, int M, int H, float *x,
+                                                                const float *w, float eps, int nst, char *xp) {
+    __shared__ float red[kResnormThreads / 64];
+    int t, chunk;
+    pack_wg(1, t, chunk);
+    if (t >= M) return;
+    const int tid = threadIdx.x;
+    float *xt = x + (size_t)t * H;
+    v4f_t v[kResnormChunks], wv[kResnormChunks];
+    float ss = 0.0f;
+#pragma unroll
+    for (int c = 0; c < kResnormChunks; c++) {
+        const int e = 4 * (tid + c * kResnormThreads);
+        v[c] = wv[c] = v4f_t{0.0f, 0.0f, 0.0f, 0.0f};
+        if (e < H) {
+            v[c] = *(const v4f_t *)(xt + e);
+            wv[c] = *(const v4f_t *)(w + e);
+            if (part) {
+                v[c] += part_sum4(part, ksplit, (size_t)M * H, (size_t)t * H + e);
+                *(v4f_t *)(xt + e) = v[c];
+            }
+        }
+        ss += v[c].x * v[c].x + v[c].y * v[c].y + v[c].z * v[c].z + v[c].w * v[c].w;
+    }
+    ss = wave_sum(ss);
+    if ((tid & 63) == 0) red[tid >> 6] = ss;
+    __syncthreads();
+    ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kResnormThreads / 64; i++) ss += red[i];
+    const float inv = 1.0f / sqrtf(ss / (float)H + eps);
+#pragma unroll
+    for (int c = 0; c < kResnormChunks; c++) {
+        const int e = 4 * (tid + c * kResnormThreads);
+        if (c * 4 * kResnormThreads >= H) break;  // uniform: shuffles below
+        float y[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) y[j] = (PRO == PRO_NORMQ0) ? v[c][j] * wv[c][j] * inv : (v[c][j] * inv) * wv[c][j];
+        pack_block8(y, e < H, xp + ((size_t)(t >> 5) * nst + (min(e, H - 4) >> 8)) * kPackRec, t, e & 255);
+    }
+}
+
+// SiLU(g) * u (silu_mul_into, model.rs:9783-9796) of the gate/up partials and
+// its Q8_0 quantization into packed records; 1024 hidden units of a token per
+// workgroup.
+__global__ __launch_bounds__(256) void k_b_silu(const float *part, int ksplit, int M, int F, int nst, char *xp) {
+    int t, chunk;
+    pack_wg((F + 1023) >> 10, t, chunk);
+    if (t >= M) return;
+    const int e = chunk * 1024 + 4 * threadIdx.x, ec = min(e, F - 4);  // F % 32 == 0
+    const size_t plane = (size_t)M * 2 * F, at = (size_t)t * 2 * F + ec;
+    const v4f_t g = part_sum4(part, ksplit, plane, at), u = part_sum4(part, ksplit, plane, at + F);
+    float y[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) y[j] = (g[j] / (1.0f + fl_expf(-g[j]))) * u[j];
+    pack_block8(y, e < F, xp + ((size_t)(t >> 5) * nst + (ec >> 8)) * kPackRec, t, e & 255);
+}
+
+// x[i] += partials of one row (part: that row of split 0; splits `plane` apart)
+__global__ __launch_bounds__(256) void k_b_residual_row(const float *part, int ksplit, size_t plane, int H, float *x) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= H) return;
+    float v = part[i];
+    for (int k = 1; k < ksplit; k++) v += part[k * plane + i];
+    x[i] += v;
 }
 
 // One workgroup: NW waves of 32 weight rows, TT tiles of 32 tokens; K in steps

@@ -239,6 +239,13 @@ struct Layer {
     float *attn_norm = nullptr, *ffn_norm = nullptr;
 };
 
+// The buffers of a pass of `cap` tokens, as offsets into one allocation.
+struct WideBufs {
+    size_t x, q, k, v, part, xp, ap, hp, split, total;
+    size_t split_plane;  // elements of one operand plane of K (and of V)
+    bool planes;         // f32 / Q8 caches: keys and values split per layer
+};
+
 struct fl_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -297,6 +304,10 @@ struct fl_ctx {
     int *vtok = nullptr, *vpos = nullptr;
     unsigned long long *vslots = nullptr;
     size_t vpart_floats = 0;
+    // wide prefill passes (allocated on the first one, for wide_cap tokens)
+    int wide_cap = 0;
+    char *wide = nullptr;
+    WideBufs wb{};
     // fl_set_option switches (measurement / testing)
     bool verify_fuse = true, verify_graph = true;
     // FL_OPT_EXACT: the decode step in the reference's floating-point order
@@ -319,6 +330,8 @@ struct fl_ctx {
 };
 
 constexpr int kVerifyMaxKsplit = 16;
+constexpr int kWideTokens = 2048;  // tokens per wide prefill pass
+constexpr size_t kWideSplitBytes = (size_t)1 << 30;  // most memory of a wide pass's f32 / Q8 key and value planes
 constexpr int kBatchRows = 2048;  // rows per GEMM of fl_op_batched_dequant_matmul (bounds its workspace)
 constexpr int kVerifyCounters = 4096;  // workgroup columns of a fused verify GEMM
 
@@ -768,6 +781,9 @@ static void model_release(fl_ctx *c) {
     c->vxsum = c->vasum = nullptr; c->vtok = c->vpos = nullptr; c->vslots = nullptr; c->vpart_floats = 0;
     c->vhq = nullptr; c->vhs = nullptr; c->vhsum = c->vcnt = nullptr;
     c->have_verify = false;
+    if (c->wide) (void)hipFree(c->wide);
+    c->wide = nullptr;
+    c->wide_cap = 0;
     c->have_cfg = c->have_weights = false;
 }
 
@@ -1917,7 +1933,7 @@ static int verify_alloc(fl_ctx *ctx) {
     ALLOC(ctx, ctx->vaq, M * qd);
     ALLOC(ctx, ctx->vas, M * (qd / 32) * 4);
     ALLOC(ctx, ctx->vasum, M * (qd / 32) * 4);
-    ALLOC(ctx, ctx->vtok, M * 4);
+    ALLOC(ctx, ctx->vtok, (size_t)kWideTokens * 4);
     ALLOC(ctx, ctx->vpos, 4);
     ALLOC(ctx, ctx->vslots, M * 8);
     ALLOC(ctx, ctx->vhq, M * F);
@@ -2141,43 +2157,37 @@ int fl_op_prefill_attention(fl_ctx *ctx, const float *q, const float *k, const f
         return fail(ctx, FL_E_INVALID, "bad prefill attention shape");
     const int G = num_heads / num_kv_heads;
     if (!attn_supported(head_dim, G)) return fail(ctx, FL_E_UNSUPPORTED, "head_dim %d / group %d", head_dim, G);
-    // queries z0 .. z0+Z-1 per launch (grid z), each attending 0..z0+z of the
-    // token-major rows; one set of split partials and counters per query
-    const int Z = std::min(seq_len, std::max(1, 1024 / num_kv_heads));
-    int ns, chmin;
-    choose_splits(seq_len, num_kv_heads, head_dim, ns, chmin);
-    ns = std::min(ns, 8);
-    int rc = ensure_part(ctx, (size_t)Z * num_kv_heads * ns * G * (head_dim + 2));
+    // keys and values as three bfloat16 operand planes, then every query in one
+    // launch
+    const size_t slots = (size_t)(seq_len + 31) / 32 * 32, kvd = (size_t)num_kv_heads * head_dim;
+    const int rc = ws_ensure(ctx, slots * kvd * 6 * 2);
     if (rc) return rc;
-    const int qd = num_heads * head_dim;
-    std::vector<int> starts;
-    for (int z0 = 0; z0 < seq_len; z0 += Z) starts.push_back(z0);
-    int *dstart = nullptr;
-    rc = dev_alloc(ctx, (void **)&dstart, starts.size() * 4);
-    if (rc) return rc;
-    hipError_t e = hipMemcpyAsync(dstart, starts.data(), starts.size() * 4, hipMemcpyHostToDevice, ctx->stream);
-    for (size_t c = 0; e == hipSuccess && c < starts.size(); c++) {
-        const int z0 = starts[c], nq = std::min(Z, seq_len - z0);
-        AttnArgs a{};
-        a.q = q + (size_t)z0 * qd;
-        a.kc = k;
-        a.vc = v;
-        a.tok_stride = (long long)num_kv_heads * head_dim;  // [token][kv_head][head_dim]
-        a.head_stride = head_dim;
-        a.posp = dstart + c;
-        a.nkv = num_kv_heads;
-        a.nsplit = ns;
-        a.chmin = chmin;
-        a.single = kAttmSingle;
-        a.part = ctx->d_part;
-        a.counters = ctx->d_counters;
-        a.out = out + (size_t)z0 * qd;
-        a.qstride = qd;
-        a.ostride = qd;
-        e = launch_attn(FL_KV_F32, head_dim, G, ctx->stream, a, nq);
-    }
+    AttwSplitArgs s{};
+    s.k = k;
+    s.v = v;
+    s.tok_stride = (long long)kvd;  // [token][kv_head][head_dim]
+    s.head_stride = head_dim;
+    s.T = seq_len;
+    s.nkv = num_kv_heads;
+    s.plane = slots * kvd;
+    s.out_stride = slots * head_dim;
+    s.ko = (uint16_t *)ctx->ws;
+    s.vo = s.ko + 3 * s.plane;
+    AttwArgs a{};
+    a.q = q;
+    a.k = s.ko;
+    a.v = s.vo;
+    a.plane = s.plane;
+    a.head_stride = s.out_stride;
+    a.slots = (int)slots;
+    a.M = seq_len;
+    a.nkv = num_kv_heads;
+    a.group = G;
+    a.qstride = num_heads * head_dim;
+    a.out = out;
+    hipError_t e = launch_attw_split(KV_F32, head_dim, ctx->stream, s);
+    if (e == hipSuccess) e = launch_attw(3, head_dim, ctx->stream, a);
     const hipError_t es = hipStreamSynchronize(ctx->stream);
-    (void)hipFree(dstart);
     HIPCHK(ctx, e);
     HIPCHK(ctx, es);
     return 0;
@@ -2206,6 +2216,27 @@ int fl_op_batched_matvec_f32in(fl_ctx *ctx, const fl_weight *w, int n_tokens, co
 // (speculative verify), nothing (prefill chunks before the last), or the key
 // / the logits of the last token only (the last prefill chunk).
 enum { VOUT_ALL = 0, VOUT_NONE = 1, VOUT_LAST_ARGMAX = 2, VOUT_LAST_LOGITS = 3 };
+
+// The Q8-input output projection (matvec_argmax_{q8_0,q4k}_preq) applies.
+static bool q8_output(const fl_ctx *ctx) {
+    const fl_weight &O = ctx->output;
+    return !ctx->tied && ((O.format == FL_Q8_0 && ctx->layer_fmt == FL_Q8_0) ||
+                          (O.format == FL_Q4K && ctx->layer_fmt == FL_Q4K));
+}
+
+// Output projection of one token's residual xt (forward_prefill returns the
+// last token's logits, model.rs:2578-3040): logits, or the greedy key in slot.
+static int last_token_output(fl_ctx *ctx, const float *xt, int out_mode, unsigned long long *slot) {
+    const fl_weight &O = ctx->tied ? ctx->embed : ctx->output;
+    const float eps = ctx->cfg.rms_norm_eps;
+    const bool q8out = q8_output(ctx);
+    const int epi = out_mode == VOUT_LAST_LOGITS ? EPI_STORE : EPI_ARGMAX;
+    if (O.format == FL_Q4K && !q8out) return fail(ctx, FL_E_UNSUPPORTED, "Q4_K output with Q8_0 layers");
+    if (q8out)
+        return launch_q8in(ctx, O, PRO_NORMQ1, epi, xt, ctx->out_norm, eps, nullptr, nullptr, nullptr, ctx->logits,
+                           slot);
+    return launch_f32in(ctx, O, 1, epi, xt, ctx->out_norm, eps, ctx->logits, slot);
+}
 
 static int enqueue_verify(fl_ctx *ctx, int M, int pos0, bool dev_pos, int out_mode = VOUT_ALL) {
     const fl_model_config &c = ctx->cfg;
@@ -2366,18 +2397,9 @@ static int enqueue_verify(fl_ctx *ctx, int M, int pos0, bool dev_pos, int out_mo
     if (out_mode == VOUT_NONE) return 0;
     // output projection + fused argmax per token (forward_greedy, model.rs:1898-1932)
     const fl_weight &O = ctx->tied ? ctx->embed : ctx->output;
-    const bool q8out = !ctx->tied && ((O.format == FL_Q8_0 && ctx->layer_fmt == FL_Q8_0) ||
-                                      (O.format == FL_Q4K && ctx->layer_fmt == FL_Q4K));
-    if (out_mode == VOUT_LAST_ARGMAX || out_mode == VOUT_LAST_LOGITS) {
-        // the last token only (forward_prefill returns its logits, model.rs:2578-3040)
-        const float *xt = xa + (size_t)(M - 1) * H;
-        const int epi = out_mode == VOUT_LAST_LOGITS ? EPI_STORE : EPI_ARGMAX;
-        if (O.format == FL_Q4K && !q8out) return fail(ctx, FL_E_UNSUPPORTED, "Q4_K output with Q8_0 layers");
-        if (q8out)
-            return launch_q8in(ctx, O, PRO_NORMQ1, epi, xt, ctx->out_norm, eps, nullptr, nullptr, nullptr, ctx->logits,
-                               ctx->vslots + (M - 1));
-        return launch_f32in(ctx, O, 1, epi, xt, ctx->out_norm, eps, ctx->logits, ctx->vslots + (M - 1));
-    }
+    const bool q8out = q8_output(ctx);
+    if (out_mode == VOUT_LAST_ARGMAX || out_mode == VOUT_LAST_LOGITS)
+        return last_token_output(ctx, xa + (size_t)(M - 1) * H, out_mode, ctx->vslots + (M - 1));
     if (!q8out && O.format != FL_F32) {
         if (O.format == FL_Q4K) return fail(ctx, FL_E_UNSUPPORTED, "Q4_K output with Q8_0 layers");
         // all M tokens in one MFMA launch (M <= 8 per launch)
@@ -2495,6 +2517,175 @@ int fl_verify(fl_ctx *ctx, const uint32_t *tokens, int n_tokens, int pos0, int32
     return 0;
 }
 
+// ---- wide prefill passes --------------------------------------------------------
+// More than kPrefillTokens prompt tokens at once: the layers as in
+// enqueue_verify, with the projections on the large-batch GEMM (its
+// activations packed by the kernels that produce them) and the many-query
+// attention.  Enqueued directly: a pass is long against its launches.
+
+static WideBufs wide_layout(const fl_ctx *ctx, int cap) {
+    const fl_model_config &c = ctx->cfg;
+    const size_t M = cap, H = c.hidden_dim, qd = (size_t)c.num_heads * c.head_dim;
+    const size_t kvd = (size_t)c.num_kv_heads * c.head_dim, F = c.intermediate_dim;
+    WideBufs b{};
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+        const size_t r = at;
+        at += (bytes + 255) & ~(size_t)255;
+        return r;
+    };
+    // partial sums of the widest GEMM of any pass of up to cap tokens
+    size_t part = 0;
+    const size_t shapes[4][2] = {{qd + 2 * kvd, H}, {H, qd}, {2 * F, H}, {H, F}};
+    for (const auto &s : shapes)
+        for (int m = 1; m <= cap; m++)
+            part = std::max(part, (size_t)bgemm_plan((int)s[0], (int)s[1], m).ksplit * m * s[0]);
+    b.x = take(M * H * 4);
+    b.q = take(M * qd * 4);
+    b.planes = ctx->kv_format == FL_KV_F32 || ctx->kv_format == FL_KV_Q8;
+    const bool staged = ctx->kv_format == FL_KV_Q8;
+    b.k = take(staged ? M * kvd * 4 : 0);
+    b.v = take(staged ? M * kvd * 4 : 0);
+    b.part = take(part * 4);
+    b.xp = take(pack_bytes(cap, (int)H));
+    b.ap = take(pack_bytes(cap, (int)qd));
+    b.hp = take(pack_bytes(cap, (int)F));
+    b.split_plane = b.planes ? (size_t)(c.max_seq_len + 31) / 32 * 32 * kvd : 0;
+    b.split = take(b.split_plane * 6 * 2);
+    b.total = at;
+    return b;
+}
+
+// Whether a prompt may run in wide passes: an fp16 cache, or an f32 / Q8 one
+// whose operand planes fit kWideSplitBytes (2-bit caches read a ring that holds
+// the newest tokens of a short pass only).
+static bool wide_possible(const fl_ctx *ctx) {
+    const fl_model_config &c = ctx->cfg;
+    if (c.hidden_dim > kResnormMaxH) return false;
+    if (ctx->kv_format == FL_KV_F16) return true;
+    return (ctx->kv_format == FL_KV_F32 || ctx->kv_format == FL_KV_Q8) &&
+           (size_t)(c.max_seq_len + 31) / 32 * 32 * c.num_kv_heads * c.head_dim * 12 <= kWideSplitBytes;
+}
+
+// Room for passes of `tokens` tokens; false if the memory is not there (the
+// caller then runs short passes).
+static bool wide_alloc(fl_ctx *ctx, int tokens) {
+    const int cap = (tokens + kPackTile - 1) / kPackTile * kPackTile;
+    if (ctx->wide_cap >= cap) return true;
+    if (ctx->wide) {
+        if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
+        (void)hipFree(ctx->wide);
+    }
+    ctx->wide = nullptr;
+    ctx->wide_cap = 0;
+    ctx->wb = wide_layout(ctx, cap);
+    if (hipMalloc((void **)&ctx->wide, ctx->wb.total) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->wide = nullptr;
+        return false;
+    }
+    ctx->wide_cap = cap;
+    return true;
+}
+
+// One wide pass of M tokens at pos0 (ids in vtok); out_mode as enqueue_verify
+// (VOUT_NONE, or the last token's key / logits, the key in vslots[0]).
+static int enqueue_wide(fl_ctx *ctx, int M, int pos0, int out_mode) {
+    const fl_model_config &c = ctx->cfg;
+    const int H = c.hidden_dim, D = c.head_dim, G = c.num_heads / c.num_kv_heads;
+    const int qd = c.num_heads * D, kvd = c.num_kv_heads * D, F = c.intermediate_dim;
+    const float eps = c.rms_norm_eps;
+    const int pro = ctx->layer_fmt == FL_Q8_0 ? PRO_NORMQ0 : PRO_NORMQ1;
+    hipStream_t st = ctx->stream;
+    const WideBufs &B = ctx->wb;
+    auto f32at = [&](size_t o) { return (float *)(ctx->wide + o); };
+    float *x = f32at(B.x), *part = f32at(B.part);
+    char *xp = ctx->wide + B.xp, *ap = ctx->wide + B.ap, *hp = ctx->wide + B.hp;
+    HIPCHK(ctx, launch_v_embed(ctx->embed.format, st, ctx->embed.desc(), ctx->vtok, M, x));
+    int ks = 0;
+    auto gemm = [&](const fl_weight &w, const char *in) {
+        const BgPlan p = bgemm_plan(w.rows, w.cols, M);
+        ks = p.ksplit;
+        return launch_bgemm(w.format, st, w.desc(), in, M, p, part);
+    };
+    for (int l = 0; l < c.num_layers; l++) {
+        Layer &L = ctx->layers[l];
+        // attention block (model.rs:2016-2311); the previous layer's down
+        // projection is added to x here
+        HIPCHK(ctx, launch_b_resnorm(pro, st, l ? part : nullptr, ks, M, H, x, L.attn_norm, eps, xp));
+        HIPCHK(ctx, gemm(L.qkv, xp));
+        AttnArgs a{};
+        kv_layer_args(ctx, l, a);
+        VgArgs::QkvPost qp{};
+        qp.nq = qd;
+        qp.nk = kvd;
+        qp.D = D;
+        qp.rope = ctx->rope;
+        qp.sin_off = (long long)c.max_seq_len * (D / 2);
+        qp.pos0p = ctx->vpos;
+        qp.Q = f32at(B.q);
+        qp.Kst = f32at(B.k);
+        qp.Vst = f32at(B.v);
+        qp.kc = const_cast<void *>(a.kc);
+        qp.vc = const_cast<void *>(a.vc);
+        qp.head_stride = a.head_stride;
+        qp.v_tblk = a.v_tblk;
+        qp.kvw = ctx->kv_format == FL_KV_F16 ? 1 : ctx->kv_format == FL_KV_F32 ? 2 : 0;
+        HIPCHK(ctx, launch_v_qkv_post(st, part, ks, M, L.qkv.rows, qp));
+        if (qp.kvw == 0) HIPCHK(ctx, launch_kv_write(ctx->kv_format, st, a, qp.Kst, qp.Vst, pos0, M, D));
+        AttwArgs w{};
+        w.q = qp.Q;
+        w.M = M;
+        w.pos0 = pos0;
+        w.nkv = c.num_kv_heads;
+        w.group = G;
+        w.qstride = qd;
+        w.xp = ap;
+        w.nst = (qd + 255) / 256;
+        if (B.planes) {
+            AttwSplitArgs s{};
+            s.k = a.kc;
+            s.v = a.vc;
+            s.ks = a.ks;
+            s.vs = a.vs;
+            s.tok_stride = D;
+            s.head_stride = a.head_stride;
+            s.v_tblk = a.v_tblk;
+            s.S = a.S;
+            s.T = pos0 + M;
+            s.nkv = c.num_kv_heads;
+            s.plane = B.split_plane;
+            s.out_stride = B.split_plane / c.num_kv_heads;
+            s.ko = (uint16_t *)(ctx->wide + B.split);
+            s.vo = s.ko + 3 * s.plane;
+            HIPCHK(ctx, launch_attw_split(ctx->kv_format, D, st, s));
+            w.k = s.ko;
+            w.v = s.vo;
+            w.plane = s.plane;
+            w.head_stride = s.out_stride;
+            w.slots = (s.T + 31) / 32 * 32;
+            HIPCHK(ctx, launch_attw(3, D, st, w));
+        } else {
+            w.k = (const uint16_t *)a.kc;
+            w.v = (const uint16_t *)a.vc;
+            w.head_stride = a.head_stride;
+            w.slots = a.S;
+            HIPCHK(ctx, launch_attw(1, D, st, w));
+        }
+        HIPCHK(ctx, gemm(L.wo, ap));
+        // FFN block (model.rs:2376-2543)
+        HIPCHK(ctx, launch_b_resnorm(pro, st, part, ks, M, H, x, L.ffn_norm, eps, xp));
+        HIPCHK(ctx, gemm(L.gu, xp));
+        HIPCHK(ctx, launch_b_silu(st, part, ks, M, F, hp));
+        HIPCHK(ctx, gemm(L.down, hp));
+    }
+    if (out_mode == VOUT_NONE) return 0;
+    // the last token's residual, then its output projection
+    const size_t row = (size_t)(M - 1) * H;
+    HIPCHK(ctx, launch_b_residual_row(st, part + row, ks, (size_t)M * H, H, x + row));
+    return last_token_output(ctx, x + row, out_mode, ctx->vslots);
+}
+
 int fl_prefill(fl_ctx *ctx, const uint32_t *tokens, int n_tokens, int pos0, float *out_logits, int32_t *out_token,
                float *out_val) {
     if (!ctx || !tokens) return fail(ctx, FL_E_INVALID, "null argument");
@@ -2516,20 +2707,31 @@ int fl_prefill(fl_ctx *ctx, const uint32_t *tokens, int n_tokens, int pos0, floa
     static const int C = measure_env("FLARE_PREFILL_TOKENS")
                              ? std::max(1, std::min(kPrefillTokens, atoi(measure_env("FLARE_PREFILL_TOKENS"))))
                              : kPrefillTokens;
-    const int nchunks = (n_tokens + C - 1) / C;
+    // prompts of more than one short pass: wide passes of up to kWideTokens
+    const bool wide = n_tokens > C && wide_possible(ctx) && wide_alloc(ctx, std::min(n_tokens, kWideTokens));
+    const int step = wide ? ctx->wide_cap : C;
+    const int nchunks = (n_tokens + step - 1) / step;
     // host copies stay alive until the final synchronisation
     std::vector<int> tk(tokens, tokens + n_tokens), pos(nchunks);
+    int slot = 0;  // of the last token's greedy key
     for (int k = 0; k < nchunks; k++) {
-        const int t0 = k * C, M = std::min(C, n_tokens - t0);
+        const int t0 = k * step, M = std::min(step, n_tokens - t0);
         pos[k] = pos0 + t0;
         HIPCHK(ctx, hipMemcpyAsync(ctx->vtok, tk.data() + t0, (size_t)M * 4, hipMemcpyHostToDevice, st));
         const int mode = k + 1 < nchunks ? VOUT_NONE : out_logits ? VOUT_LAST_LOGITS : VOUT_LAST_ARGMAX;
-        rc = run_verify_pass(ctx, M, &pos[k], mode);
+        if (M > C) {
+            HIPCHK(ctx, hipMemcpyAsync(ctx->vpos, &pos[k], 4, hipMemcpyHostToDevice, st));
+            if (mode != VOUT_NONE) HIPCHK(ctx, hipMemsetAsync(ctx->vslots, 0, 8, st));
+            rc = enqueue_wide(ctx, M, pos[k], mode);
+            slot = 0;
+        } else {
+            rc = run_verify_pass(ctx, M, &pos[k], mode);
+            slot = M - 1;
+        }
         if (rc) return rc;
     }
-    const int Mlast = n_tokens - (nchunks - 1) * C;
     unsigned long long key = 0;
-    HIPCHK(ctx, hipMemcpyAsync(&key, ctx->vslots + (Mlast - 1), 8, hipMemcpyDeviceToHost, st));
+    HIPCHK(ctx, hipMemcpyAsync(&key, ctx->vslots + slot, 8, hipMemcpyDeviceToHost, st));
     if (out_logits)
         HIPCHK(ctx, hipMemcpyAsync(out_logits, ctx->logits, (size_t)ctx->cfg.vocab_size * 4, hipMemcpyDeviceToHost, st));
     HIPCHK(ctx, hipStreamSynchronize(st));

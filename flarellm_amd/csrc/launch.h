@@ -10,6 +10,7 @@
 #include <utility>
 
 #include "attn_kernels.h"
+#include "attw_args.h"
 #include "bgemm_args.h"
 #include "mvs_kernels.h"
 #include "verify_args.h"
@@ -139,6 +140,10 @@ hipError_t launch_mvs_gu_q4k(const MvsPlan &p, hipStream_t st, const MvsArgs &a)
 enum KvFmt { KV_F32 = 0, KV_F16 = 1, KV_Q8 = 2, KV_KIVI = 3 };  // == FL_KV_*
 hipError_t launch_attn(int kvfmt, int D, int G, hipStream_t st, const AttnArgs &a, int nq = 1);
 hipError_t launch_attq(int D, int G, hipStream_t st, const AttnArgs &a);
+// attention of many queries over one (binary16) or three (bfloat16) operand
+// planes, and the split of f32 / Q8 keys and values into the latter (attw.hip)
+hipError_t launch_attw(int planes, int D, hipStream_t st, const AttwArgs &a);
+hipError_t launch_attw_split(int kvfmt, int D, hipStream_t st, const AttwSplitArgs &a);
 // fused QKV matvec + decode attention (fused.hip): nqwg QKV workgroups (a
 // multiple of a.nkv) of nt threads, then a.nsplit * a.nkv attention ones
 hipError_t launch_qkv_attm(int fmt, const MvsPlan &p, int rx, int D, int G, int nt, hipStream_t st,
@@ -181,6 +186,10 @@ struct BgPlan {
 BgPlan bgemm_plan(int rows, int cols, int M);
 hipError_t launch_bgemm(int fmt, hipStream_t st, const WDesc &W, const char *xp, int M, const BgPlan &p, float *part);
 hipError_t launch_quant_pack(hipStream_t st, const float *x, int M, int K, char *xp);
+hipError_t launch_b_resnorm(int pro, hipStream_t st, const float *part, int ksplit, int M, int H, float *x,
+                            const float *w, float eps, char *xp);
+hipError_t launch_b_residual_row(hipStream_t st, const float *part, int ksplit, size_t plane, int H, float *x);
+hipError_t launch_b_silu(hipStream_t st, const float *part, int ksplit, int M, int F, char *xp);
 
 // speculative verify (verify.hip)
 hipError_t launch_vgemm(int fmt, hipStream_t st, const VgArgs &a);

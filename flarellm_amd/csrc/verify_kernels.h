@@ -1009,9 +1009,6 @@ __global__ __launch_bounds__(256) void k_v_store(const float *part, int ksplit, 
 // 5581-5640 / 7456-7477).  Thread i holds elements 4i..4i+3 of every
 // 4096-element chunk in registers (H <= kResnormMaxH), so 8 lanes form one
 // 32-block; the norm weights load before the reduction.
-constexpr int kResnormThreads = 1024;
-constexpr int kResnormChunks = 4;
-constexpr int kResnormMaxH = 4 * kResnormThreads * kResnormChunks;
 template <int PRO>
 __global__ __launch_bounds__(kResnormThreads) void k_v_resnorm(const float *part, int ksplit, int M, int H, float *x,
                                                                 const float *w, float eps, int8_t *q, float *s,

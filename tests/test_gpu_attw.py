@@ -1,0 +1,105 @@
+"""Many-query attention (k_attw): prefill_attention_gpu at the edges of its
+tiles (32 queries per item, 4 items per workgroup, 64 keys per iteration), and
+wide prefill passes against the same prompt in short ones."""
+import numpy as np
+import pytest
+
+from flarellm_amd import FL_KV_F16, FL_KV_F32, FL_KV_Q8, FL_Q4K, FL_Q6K, FL_Q8_0
+from flarellm_amd import synth as S
+
+pytestmark = pytest.mark.gpu
+
+
+def _reference(q, k, v, nh, nkv, hd):
+    """float64 causal attention and sum_t p_t |v_t| of each output."""
+    T, g = q.shape[0], nh // nkv
+    q, k, v = (a.astype(np.float64).reshape(T, -1, hd) for a in (q, k, v))
+    out, mag = np.empty_like(q), np.empty_like(q)
+    top = np.zeros((T, nh, 1))
+    for h in range(nh):
+        s = q[:, h] @ k[:, h // g].T / np.sqrt(hd)
+        s[np.triu_indices(T, 1)] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        p /= p.sum(1, keepdims=True)
+        out[:, h], mag[:, h] = p @ v[:, h // g], p @ np.abs(v[:, h // g])
+        top[:, h, 0] = np.where(np.isfinite(s), np.abs(s), 0).max(1)
+    return out.reshape(T, -1), mag.reshape(T, -1), np.repeat(top, hd, 2).reshape(T, -1)
+
+
+def _check(backend, nh, nkv, hd, T, edit=None):
+    import torch
+
+    print(f"[attw] heads={nh}/{nkv} D={hd} T={T}", flush=True)
+    q = S.normal(T + hd, 0, T * nh * hd).reshape(T, -1)
+    k = S.normal(T + hd, 1 << 40, T * nkv * hd).reshape(T, -1)
+    v = S.normal(T + hd, 2 << 40, T * nkv * hd).reshape(T, -1)
+    if edit is not None:
+        edit(q, k, v)
+    got = backend.prefill_attention_gpu(*(torch.from_numpy(a).cuda() for a in (q, k, v)), T, nh, nkv, hd).cpu().numpy()
+    want, mag, top = _reference(q, k, v, nh, nkv, hd)
+    # a score's error is at most ~(hd + 16) 2^-24 of |q||k| <= the largest
+    # |score| here times sqrt(hd); p's relative error is the same absolute
+    # amount, and the sums over T keys add sqrt(T) 2^-24
+    sq = np.linalg.norm(q.reshape(T, nh, hd).astype(np.float64), axis=2).max() * \
+        np.linalg.norm(k.reshape(T, nkv, hd).astype(np.float64), axis=2).max() / np.sqrt(hd)
+    bound = (4 * np.sqrt(hd) * sq + 4 * np.sqrt(T) + 16) * 2.0 ** -24 * mag
+    assert (np.abs(got - want) <= bound + 1e-30).all(), float((np.abs(got - want) / (bound + 1e-30)).max())
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(1, 1, 64), (6, 3, 128), (9, 3, 64), (16, 4, 128), (16, 2, 64)])
+@pytest.mark.parametrize("T", [1, 31, 32, 33, 64, 65, 97, 129, 300])
+def test_edges(backend, nh, nkv, hd, T):
+    _check(backend, nh, nkv, hd, T)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+def test_values(backend, hd):
+    """Zero queries (a plain mean), large scores (one key takes all), values of
+    very different size."""
+
+    def edit(q, k, v):
+        q[3] = 0.0
+        q[40:50] *= 30.0
+        v[::7] *= 1e4
+        v[5] *= 1e-6
+
+    _check(backend, 8, 2, hd, 100, edit)
+
+
+@pytest.mark.parametrize("kv", [FL_KV_F16, FL_KV_Q8, FL_KV_F32])
+@pytest.mark.parametrize("fmt,hd,pos0,n", [(FL_Q8_0, 64, 0, 65), (FL_Q4K, 128, 37, 200), (FL_Q8_0, 128, 3, 2150)])
+def test_wide_prefill_matches_short_passes(backend, kv, fmt, hd, pos0, n):
+    """The last token's logits and the cache a wide prefill leaves (through a
+    decode step after it) against the same tokens in 16-token calls.  The two
+    round differently, and requantized activations turn a last bit into a code
+    step: 1 % of the largest logit, as the prefill tests hold the oracle to."""
+    print(f"[wide] kv={kv} fmt={fmt} D={hd} pos0={pos0} n={n}", flush=True)
+    spec = S.tiny_spec(fmt, embed_fmt=FL_Q6K if fmt == FL_Q4K else None, output_fmt=FL_Q6K if fmt == FL_Q4K else None,
+                       heads=4, kv_heads=2, head_dim=hd, hidden=512, max_seq=pos0 + n + 8)
+    model = S.make_model(spec, seed=9)
+    toks = S.random_tokens(4, pos0 + n, spec.vocab)
+    backend.init_gpu_kv_cache(spec, kv)
+    backend.upload_weights_to_gpu(model)
+    res = []
+    for step in (n, 16):
+        backend.reset()
+        if pos0:
+            backend.forward_prefill(toks[:pos0], 0, logits=False)
+        for t in range(pos0, pos0 + n, step):
+            logits, tok, val = backend.forward_prefill(toks[t:min(t + step, pos0 + n)], t)
+        assert tok == int(np.argmax(logits)) and val == logits[tok]
+        res.append((logits, backend.forward_single_token_gpu(1, pos0 + n)))
+    for a, b in zip(*res):
+        assert np.abs(a - b).max() <= 0.01 * np.abs(b).max()
+
+
+def test_wide_prefill_greedy_key(backend):
+    """Without logits the wide pass returns the fused argmax of the same row."""
+    spec = S.tiny_spec(FL_Q8_0, max_seq=256)
+    backend.init_gpu_kv_cache(spec, FL_KV_F16)
+    backend.upload_weights_to_gpu(S.make_model(spec, seed=2))
+    toks = S.random_tokens(5, 130, spec.vocab)
+    logits, tok, val = backend.forward_prefill(toks, 0)
+    backend.reset()
+    none, tok2, val2 = backend.forward_prefill(toks, 0, logits=False)
+    assert none is None and tok2 == tok and val2 == val
