@@ -35,8 +35,11 @@ hipError_t launch_tt(int tt, hipStream_t st, const BgArgs &a) {
 // and round of the chip on MI355X (28672 x 4096 Q4_K, 2048 tokens): 2.9, 4.3,
 // 5.4 and 7.0 us with 1, 2, 3 and 4 token tiles.  K is split where tiles alone
 // leave CUs idle; the split's partial sums cost a write, a read (4 TB/s
-// together) and a launch.
-BgPlan bgemm_plan(int rows, int cols, int M) {
+// together) and a launch.  Q8_0 sums every 32-block straight into its output,
+// so a split holds at most kQ8Steps steps (7168 values: 1.4e-7 against 64 bits
+// where 14336 in one chain had 2.0e-7).
+constexpr int kQ8Steps = 28;
+BgPlan bgemm_plan(int fmt, int rows, int cols, int M) {
     static const double step_us[5] = {0, 2.9, 4.3, 5.4, 7.0};
     const int tiles = (M + kPackTile - 1) / kPackTile, nst = (cols + 255) / 256;
     BgPlan best{};
@@ -51,7 +54,7 @@ BgPlan bgemm_plan(int rows, int cols, int M) {
                 p.nrt = (rows + 32 * nw - 1) / (32 * nw);
                 p.chunk = (nst + want - 1) / want;
                 p.ksplit = (nst + p.chunk - 1) / p.chunk;
-                if (p.ksplit != want) continue;
+                if (p.ksplit != want || (fmt == F_Q8_0 && p.chunk > kQ8Steps)) continue;
                 const long long wgs = (long long)p.nrt * p.ntt * p.ksplit, slots = nw == 8 ? 256 : 512;
                 double us = (double)((wgs + slots - 1) / slots) * p.chunk * step_us[tt];
                 if (p.ksplit > 1) us += 4.0 + 2.0 * p.ksplit * M * (double)rows * 4 / 4e6;

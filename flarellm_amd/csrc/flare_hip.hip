@@ -2111,7 +2111,7 @@ int fl_op_batched_dequant_matmul(fl_ctx *ctx, const fl_weight *w, const float *i
         // then one GEMM per kBatchRows rows
         for (int b0 = 0; b0 < batch && e == hipSuccess; b0 += kBatchRows) {
             const int n = std::min(kBatchRows, batch - b0);
-            const BgPlan p = bgemm_plan(w->rows, cols, n);
+            const BgPlan p = bgemm_plan(w->format, w->rows, cols, n);
             const size_t xb = pack_bytes(n, cols);
             const int rc = ws_ensure(ctx, xb + (p.ksplit > 1 ? (size_t)p.ksplit * n * w->rows * 4 : 0));
             if (rc) return rc;
@@ -2539,7 +2539,7 @@ static WideBufs wide_layout(const fl_ctx *ctx, int cap) {
     const size_t shapes[4][2] = {{qd + 2 * kvd, H}, {H, qd}, {2 * F, H}, {H, F}};
     for (const auto &s : shapes)
         for (int m = 1; m <= cap; m++)
-            part = std::max(part, (size_t)bgemm_plan((int)s[0], (int)s[1], m).ksplit * m * s[0]);
+            part = std::max(part, (size_t)bgemm_plan(ctx->layer_fmt, (int)s[0], (int)s[1], m).ksplit * m * s[0]);
     b.x = take(M * H * 4);
     b.q = take(M * qd * 4);
     b.planes = ctx->kv_format == FL_KV_F32 || ctx->kv_format == FL_KV_Q8;
@@ -2604,7 +2604,7 @@ static int enqueue_wide(fl_ctx *ctx, int M, int pos0, int out_mode) {
     HIPCHK(ctx, launch_v_embed(ctx->embed.format, st, ctx->embed.desc(), ctx->vtok, M, x));
     int ks = 0;
     auto gemm = [&](const fl_weight &w, const char *in) {
-        const BgPlan p = bgemm_plan(w.rows, w.cols, M);
+        const BgPlan p = bgemm_plan(w.format, w.rows, w.cols, M);
         ks = p.ksplit;
         return launch_bgemm(w.format, st, w.desc(), in, M, p, part);
     };

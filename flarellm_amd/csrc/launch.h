@@ -183,7 +183,7 @@ constexpr int kBgMaxSplit = 32;
 struct BgPlan {
     int tt, nw, nrt, ntt, ksplit, chunk;
 };
-BgPlan bgemm_plan(int rows, int cols, int M);
+BgPlan bgemm_plan(int fmt, int rows, int cols, int M);
 hipError_t launch_bgemm(int fmt, hipStream_t st, const WDesc &W, const char *xp, int M, const BgPlan &p, float *part);
 hipError_t launch_quant_pack(hipStream_t st, const float *x, int M, int K, char *xp);
 hipError_t launch_b_resnorm(int pro, hipStream_t st, const float *part, int ksplit, int M, int H, float *x,

@@ -212,3 +212,27 @@ def test_verify_graph_replays_match_eager(backend, oracle, kv, monkeypatch):
             # eager work between replays (rewrites the first slots it verified)
             backend.forward_greedy(int(drafts[0]), pos)
             backend.sync()
+
+
+@pytest.mark.parametrize("fmt,rows,cols,M", [
+    (FL_Q6K, 17, 256, 2), (FL_Q6K, 33, 512, 3), (FL_Q6K, 4100, 1024, 8), (FL_Q6K, 130, 2304, 7),
+    (FL_Q6K, 300, 4864, 8), (FL_Q8_0, 15, 32, 5), (FL_Q8_0, 33, 96, 8), (FL_Q8_0, 513, 1056, 6),
+    (FL_Q8_0, 130, 2080, 2), (FL_Q8_0, 100, 5088, 8),
+])
+def test_multi_token_logits_tile_edges(backend, oracle, fmt, rows, cols, M):
+    """k_mvo at its edges: ragged rows, a K that gives some of the waves of a
+    tile no unit, rows that end inside one, the longest K (two launches), the
+    MFMA's zero rows (M < 8).  float64 reference; each output sums K exact
+    products of weights and 22-bit activations: 2^-22 per product and
+    (K / 16 + 16) roundings of 2^-24, all of sum |w||x|."""
+    import torch
+
+    print(f"[mvo] fmt={fmt} {rows}x{cols} M={M}", flush=True)
+    w = S.quantize(S.normal(rows + cols, 0, rows * cols, 0, 0.02).reshape(rows, cols), fmt)
+    W = backend.upload(S.QWeight(w, fmt, rows, cols))
+    x = S.normal(cols + M, 1 << 40, M * cols).reshape(M, cols)
+    got = backend.batched_matvec_f32in(W, torch.from_numpy(x).cuda()).cpu().numpy()
+    W.free()
+    wd = oracle.dequant(w, fmt, rows, cols).astype(np.float64)
+    bound = (2.0 ** -22 + (cols / 16 + 16) * 2.0 ** -24) * (np.abs(x) @ np.abs(wd).T)
+    assert (np.abs(got - x.astype(np.float64) @ wd.T) <= bound).all()
