@@ -167,13 +167,23 @@ constexpr int kEmbedThreads = 1024;
 template <int FMT>
 // x == nullptr: the embedding row is already in the residual buffer (a caller
 // that passes the f32 embedding, forward_single_token_gpu model.rs:555).
+// host != nullptr: the step's (token, position) in pinned host memory, read
+// over the bus instead of being copied to the device first; key (optional):
+// the argmax slot of a step that stores its logits, cleared here.
 __global__ __launch_bounds__(kEmbedThreads) void k_embed(WDesc E, DevState *st, int *tokens, float *x, const float *rope,
-                                                   long long sin_off, int half, float *rope_cur) {
+                                                   long long sin_off, int half, float *rope_cur, const int *host,
+                                                   unsigned long long *key) {
     __shared__ int tok_s, step_s;
     if (threadIdx.x == 0) {
-        const int s = st->step;
+        if (key) *key = 0ull;
+        int s = host ? 0 : st->step;
         int tok;
-        if (s < st->n_prompt) {
+        if (host) {
+            tok = __hip_atomic_load(host, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            s = __hip_atomic_load(host + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            tokens[s] = tok;
+            st->n_prompt = s + 1;
+        } else if (s < st->n_prompt) {
             tok = tokens[s];
         } else {
             tok = (int)key_index(st->argmax);
@@ -284,6 +294,10 @@ struct fl_ctx {
     float *x = nullptr, *qkv = nullptr, *attn = nullptr, *logits = nullptr;
     float *bench_out = nullptr;  // output of fl_bench_layer_kernel launches
     long long *bench_trace = nullptr;  // attention phase timestamps (FLARE_ATTN_TRACE builds)
+    char *hpin = nullptr;              // pinned host memory, in parts:
+    int *hstep = nullptr;              //   (token, position) of a directly enqueued step
+    char *hstage = nullptr;            //   fl_gqa_from_cache, fl_verify
+    char *hlogits = nullptr;           //   logits and their key
     float *rope_cur = nullptr;         // RoPE (cos, sin) of the step in flight [D]
     int8_t *aq = nullptr, *hq = nullptr;
     float *as = nullptr, *hs = nullptr;
@@ -685,6 +699,12 @@ static int ws_ensure(fl_ctx *ctx, size_t bytes) {
     return 0;
 }
 
+// The key slot after the logits (one copy reads both back).
+static size_t logits_key_off(const fl_ctx *ctx) { return ((size_t)ctx->cfg.vocab_size * 4 + 15) & ~(size_t)15; }
+static unsigned long long *logits_key(fl_ctx *ctx) {
+    return (unsigned long long *)((char *)ctx->logits + logits_key_off(ctx));
+}
+
 // =====================================================================
 // C-ABI
 // =====================================================================
@@ -774,13 +794,17 @@ static void model_release(fl_ctx *c) {
     c->probe_layer = -1;
     c->probe_host = nullptr;
     void *vp[] = {c->vx, c->vx2, c->vq, c->vk, c->vv, c->vpart, c->vxq, c->vaq, c->vxs, c->vas, c->vxsum, c->vasum,
-                  c->vtok, c->vpos, c->vslots, c->vhq, c->vhs, c->vhsum, c->vcnt};
+                  c->vpos, c->vslots, c->vhq, c->vhs, c->vhsum, c->vcnt};
     for (void *p : vp)
         if (p) (void)hipFree(p);
     c->vx = c->vx2 = c->vq = c->vk = c->vv = c->vpart = nullptr; c->vxq = c->vaq = nullptr; c->vxs = c->vas = nullptr;
     c->vxsum = c->vasum = nullptr; c->vtok = c->vpos = nullptr; c->vslots = nullptr; c->vpart_floats = 0;
     c->vhq = nullptr; c->vhs = nullptr; c->vhsum = c->vcnt = nullptr;
     c->have_verify = false;
+    if (c->hpin) (void)hipHostFree(c->hpin);
+    c->hpin = nullptr;
+    c->hstep = nullptr;
+    c->hstage = c->hlogits = nullptr;
     if (c->wide) (void)hipFree(c->wide);
     c->wide = nullptr;
     c->wide_cap = 0;
@@ -1126,7 +1150,13 @@ int fl_model_init(fl_ctx *ctx, const fl_model_config *cfg, int kv_format) {
     ALLOC(ctx, ctx->hq, F);
     ALLOC(ctx, ctx->hs, F / 32 * 4);
     ALLOC(ctx, ctx->hsum, F / 32 * 4);
-    ALLOC(ctx, ctx->logits, (size_t)c.vocab_size * 4);
+    ALLOC(ctx, ctx->logits, logits_key_off(ctx) + 16);
+    // pinned: a step's token and position, small transfers, the logits read back
+    const size_t stage = std::max<size_t>(512, (qd + 16) * 4);
+    HIPCHK(ctx, hipHostMalloc((void **)&ctx->hpin, 64 + stage + 64 + logits_key_off(ctx) + 16, hipHostMallocDefault));
+    ctx->hstep = (int *)ctx->hpin;
+    ctx->hstage = ctx->hpin + 64;
+    ctx->hlogits = ctx->hstage + ((stage + 63) & ~(size_t)63);
     ALLOC(ctx, ctx->bench_out, std::max({(size_t)c.vocab_size, H, qd + 2 * kvd, 2 * F}) * 4);
     ALLOC(ctx, ctx->bench_trace, (64 + 3072) * 8);
     ALLOC(ctx, ctx->rope_cur, (size_t)c.head_dim * 4);
@@ -1332,6 +1362,30 @@ static void kv_layer_args(fl_ctx *ctx, int l, AttnArgs &a) {
     }
 }
 
+static void unpack_key(unsigned long long k, int32_t *tok, float *val);
+
+// Read the logits back through the pinned buffer (waits for the stream), with
+// their first maximum: from the key, or without one by a scan.
+static int read_logits(fl_ctx *ctx, bool key, float *out, int32_t *out_token, float *out_val) {
+    const size_t n = (size_t)ctx->cfg.vocab_size, off = logits_key_off(ctx);
+    HIPCHK(ctx, hipMemcpyAsync(ctx->hlogits, ctx->logits, off + 8, hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    std::memcpy(out, ctx->hlogits, n * 4);
+    int32_t bi = 0;
+    float bv = -INFINITY;
+    if (key) {
+        unsigned long long k;
+        std::memcpy(&k, ctx->hlogits + off, 8);
+        if (k) unpack_key(k, &bi, &bv);
+    } else {
+        for (size_t i = 0; i < n; i++)
+            if (out[i] > bv) { bv = out[i]; bi = (int32_t)i; }
+    }
+    if (out_token) *out_token = bi;
+    if (out_val) *out_val = bv;
+    return 0;
+}
+
 // Enqueue one decode step (kernels only; no host synchronisation).
 // Attention of layer l over the head-major cache [kv_head][slot][head_dim]
 // (q from the fused QKV output, RoPE already applied by its epilogue).
@@ -1491,7 +1545,10 @@ static int launch_qkv_attention(fl_ctx *ctx, const fl_weight &w, const float *no
 }
 
 // x_given: the caller has put the step's f32 embedding row into ctx->x.
-static int enqueue_step(fl_ctx *ctx, bool want_logits, bool x_given = false) {
+// host_step: (token, position) come from ctx->hstep, and the logits' argmax key
+// goes to logits_key (not in the reference-order mode, whose output kernel
+// stores only).
+static int enqueue_step(fl_ctx *ctx, bool want_logits, bool x_given = false, bool host_step = false) {
     const fl_model_config &c = ctx->cfg;
     if (ctx->exact && ctx->kv_format != FL_KV_F32 && ctx->kv_format != FL_KV_F16)
         return fail(ctx, FL_E_UNSUPPORTED, "FL_OPT_EXACT needs an F32 or F16 KV cache (the reference's forms)");
@@ -1499,11 +1556,14 @@ static int enqueue_step(fl_ctx *ctx, bool want_logits, bool x_given = false) {
     const float eps = c.rms_norm_eps;
     const int norm_pro = ctx->layer_fmt == FL_Q8_0 ? PRO_NORMQ0 : PRO_NORMQ1;
     const long long sin_off = (long long)c.max_seq_len * (c.head_dim / 2);
+    const int *hs = host_step ? ctx->hstep : nullptr;
+    unsigned long long *key = host_step && want_logits && !ctx->exact ? logits_key(ctx) : nullptr;
+    const int out_epi = !want_logits ? EPI_ARGMAX : key ? EPI_STORE_ARGMAX : EPI_STORE;
     switch (ctx->embed.format) {
-    case FL_Q8_0: hipLaunchKernelGGL(k_embed<F_Q8_0>, dim3(1), dim3(kEmbedThreads), 0, ctx->stream, ctx->embed.desc(), ctx->st, ctx->tokens, x_given ? nullptr : ctx->x, ctx->rope, sin_off, c.head_dim / 2, ctx->rope_cur); break;
-    case FL_Q6K: hipLaunchKernelGGL(k_embed<F_Q6K>, dim3(1), dim3(kEmbedThreads), 0, ctx->stream, ctx->embed.desc(), ctx->st, ctx->tokens, x_given ? nullptr : ctx->x, ctx->rope, sin_off, c.head_dim / 2, ctx->rope_cur); break;
-    case FL_Q4K: hipLaunchKernelGGL(k_embed<F_Q4K>, dim3(1), dim3(kEmbedThreads), 0, ctx->stream, ctx->embed.desc(), ctx->st, ctx->tokens, x_given ? nullptr : ctx->x, ctx->rope, sin_off, c.head_dim / 2, ctx->rope_cur); break;
-    default: hipLaunchKernelGGL(k_embed<F_F32>, dim3(1), dim3(kEmbedThreads), 0, ctx->stream, ctx->embed.desc(), ctx->st, ctx->tokens, x_given ? nullptr : ctx->x, ctx->rope, sin_off, c.head_dim / 2, ctx->rope_cur); break;
+    case FL_Q8_0: hipLaunchKernelGGL(k_embed<F_Q8_0>, dim3(1), dim3(kEmbedThreads), 0, ctx->stream, ctx->embed.desc(), ctx->st, ctx->tokens, x_given ? nullptr : ctx->x, ctx->rope, sin_off, c.head_dim / 2, ctx->rope_cur, hs, key); break;
+    case FL_Q6K: hipLaunchKernelGGL(k_embed<F_Q6K>, dim3(1), dim3(kEmbedThreads), 0, ctx->stream, ctx->embed.desc(), ctx->st, ctx->tokens, x_given ? nullptr : ctx->x, ctx->rope, sin_off, c.head_dim / 2, ctx->rope_cur, hs, key); break;
+    case FL_Q4K: hipLaunchKernelGGL(k_embed<F_Q4K>, dim3(1), dim3(kEmbedThreads), 0, ctx->stream, ctx->embed.desc(), ctx->st, ctx->tokens, x_given ? nullptr : ctx->x, ctx->rope, sin_off, c.head_dim / 2, ctx->rope_cur, hs, key); break;
+    default: hipLaunchKernelGGL(k_embed<F_F32>, dim3(1), dim3(kEmbedThreads), 0, ctx->stream, ctx->embed.desc(), ctx->st, ctx->tokens, x_given ? nullptr : ctx->x, ctx->rope, sin_off, c.head_dim / 2, ctx->rope_cur, hs, key); break;
     }
     HIPCHK(ctx, hipGetLastError());
     const size_t H = c.hidden_dim, nq = (size_t)c.num_heads * hd, nk = (size_t)c.num_kv_heads * hd;
@@ -1617,8 +1677,8 @@ static int enqueue_step(fl_ctx *ctx, bool want_logits, bool x_given = false) {
                                       (O.format == FL_Q4K && ctx->layer_fmt == FL_Q4K));
     int rc;
     if (q8out) {
-        rc = launch_q8in(ctx, O, PRO_NORMQ1, want_logits ? EPI_STORE : EPI_ARGMAX, ctx->x, ctx->out_norm, eps,
-                         nullptr, nullptr, nullptr, ctx->logits, &ctx->st->argmax);
+        rc = launch_q8in(ctx, O, PRO_NORMQ1, out_epi, ctx->x, ctx->out_norm, eps, nullptr, nullptr, nullptr, ctx->logits,
+                         key ? key : &ctx->st->argmax);
     } else if (ctx->exact) {
         // rmsnorm_into, then matvec_argmax_f32 / matvec_into over the dequantized weight
         HIPCHK(ctx, launch_rmsnorm_seq(ctx->stream, ctx->x, ctx->out_norm, c.hidden_dim, eps, ctx->seq_xn));
@@ -1627,8 +1687,7 @@ static int enqueue_step(fl_ctx *ctx, bool want_logits, bool x_given = false) {
         rc = 0;
     } else {
         if (O.format == FL_Q4K) return fail(ctx, FL_E_UNSUPPORTED, "Q4_K output with Q8_0 layers");
-        rc = launch_f32in(ctx, O, 1, want_logits ? EPI_STORE : EPI_ARGMAX, ctx->x, ctx->out_norm, eps, ctx->logits,
-                          &ctx->st->argmax);
+        rc = launch_f32in(ctx, O, 1, out_epi, ctx->x, ctx->out_norm, eps, ctx->logits, key ? key : &ctx->st->argmax);
     }
     return rc;
 }
@@ -1681,49 +1740,36 @@ static int decode_step(fl_ctx *ctx, uint32_t token, const float *embedding, int 
         return fail(ctx, FL_E_INVALID, "pos %d outside the KV cache (max_seq_len %d)", pos, c.max_seq_len);
     if ((int)token >= c.vocab_size) return fail(ctx, FL_E_INVALID, "token %u >= vocab", token);
     const int tok = (int)token;
-    DevState hs{};
-    hs.step = pos;
-    hs.pos = pos;
-    hs.n_prompt = pos + 1;
-    HIPCHK(ctx, hipMemcpyAsync(ctx->tokens + pos, &tok, 4, hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(ctx, hipMemcpyAsync(ctx->st, &hs, sizeof hs, hipMemcpyHostToDevice, ctx->stream));
     if (embedding)
         HIPCHK(ctx, hipMemcpyAsync(ctx->x, embedding, (size_t)c.hidden_dim * 4, hipMemcpyHostToDevice, ctx->stream));
-    if (out_logits || embedding || ctx->probe_layer >= 0) {
+    const bool direct = out_logits || embedding || ctx->probe_layer >= 0;
+    if (direct) {
         // enqueued directly: the captured step dequantizes the token's row
-        // (and carries no probe copies)
-        int rc = enqueue_step(ctx, out_logits != nullptr, embedding != nullptr);
+        // (and carries no probe copies).  Every call waits for the stream, so
+        // the pinned words are free to write.
+        ctx->hstep[0] = tok;
+        ctx->hstep[1] = pos;
+        int rc = enqueue_step(ctx, out_logits != nullptr, embedding != nullptr, true);
         if (rc) return rc;
     } else {
+        DevState hs{};
+        hs.step = pos;
+        hs.pos = pos;
+        hs.n_prompt = pos + 1;
+        HIPCHK(ctx, hipMemcpyAsync(ctx->tokens + pos, &tok, 4, hipMemcpyHostToDevice, ctx->stream));
+        HIPCHK(ctx, hipMemcpyAsync(ctx->st, &hs, sizeof hs, hipMemcpyHostToDevice, ctx->stream));
         int rc = ensure_graph(ctx);
         if (!rc) rc = launch_step(ctx);
         if (rc) return rc;
     }
-    DevState out{};
-    HIPCHK(ctx, hipMemcpyAsync(&out, ctx->st, sizeof out, hipMemcpyDeviceToHost, ctx->stream));
-    if (out_logits)
-        HIPCHK(ctx, hipMemcpyAsync(out_logits, ctx->logits, (size_t)c.vocab_size * 4, hipMemcpyDeviceToHost,
-                                   ctx->stream));
     if (ctx->probe_layer >= 0 && ctx->probe_host)
         HIPCHK(ctx, hipMemcpyAsync(ctx->probe_host, ctx->probe_dev, ctx->probe_bytes, hipMemcpyDeviceToHost,
                                    ctx->stream));
+    if (out_logits) return read_logits(ctx, !ctx->exact, out_logits, out_token, out_val);
+    DevState out{};
+    HIPCHK(ctx, hipMemcpyAsync(&out, ctx->st, sizeof out, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    if (out_logits) {
-        int bi = 0;
-        float bv = -INFINITY;
-        for (int i = 0; i < c.vocab_size; i++)
-            if (out_logits[i] > bv) { bv = out_logits[i]; bi = i; }
-        if (out_token) *out_token = bi;
-        if (out_val) *out_val = bv;
-    } else {
-        const unsigned long long k = out.argmax;
-        if (out_token) *out_token = (int32_t)(0xFFFFFFFFu - (uint32_t)(k & 0xFFFFFFFFull));
-        uint32_t u = (uint32_t)(k >> 32);
-        u = (u & 0x80000000u) ? (u & 0x7FFFFFFFu) : ~u;
-        float v;
-        std::memcpy(&v, &u, 4);
-        if (out_val) *out_val = v;
-    }
+    unpack_key(out.argmax, out_token, out_val);
     return 0;
 }
 
@@ -1862,13 +1908,16 @@ int fl_gqa_from_cache(fl_ctx *ctx, int layer, const float *q, int seq_len, float
     if (layer < 0 || layer >= c.num_layers) return fail(ctx, FL_E_INVALID, "layer %d", layer);
     if (seq_len <= 0 || seq_len > c.max_seq_len) return fail(ctx, FL_E_INVALID, "seq_len %d", seq_len);
     const size_t qd = (size_t)c.num_heads * c.head_dim;
-    HIPCHK(ctx, hipMemcpyAsync(ctx->qkv, q, qd * 4, hipMemcpyHostToDevice, ctx->stream));
+    // the query and, behind it, the position in one copy through the pinned
+    // buffer (every call waits for the stream)
+    std::memcpy(ctx->hstage, q, qd * 4);
     const int pos = seq_len - 1;
-    HIPCHK(ctx, hipMemcpyAsync(ctx->d_pos, &pos, 4, hipMemcpyHostToDevice, ctx->stream));
+    std::memcpy(ctx->hstage + qd * 4, &pos, 4);
+    HIPCHK(ctx, hipMemcpyAsync(ctx->qkv, ctx->hstage, qd * 4 + 4, hipMemcpyHostToDevice, ctx->stream));
     AttnArgs a{};
     kv_layer_args(ctx, layer, a);
     a.q = ctx->qkv;
-    a.posp = ctx->d_pos;
+    a.posp = (const int *)(ctx->qkv + qd);
     a.nsplit = ctx->nsplit;
     a.chmin = ctx->chmin;
     a.single = ctx->single;
@@ -1878,8 +1927,9 @@ int fl_gqa_from_cache(fl_ctx *ctx, int layer, const float *q, int seq_len, float
     a.out = ctx->attn;
     int rc = launch_attention(ctx, ctx->kv_format, c.head_dim, c.num_heads / c.num_kv_heads, a);
     if (rc) return rc;
-    HIPCHK(ctx, hipMemcpyAsync(out, ctx->attn, qd * 4, hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(ctx, hipMemcpyAsync(ctx->hstage, ctx->attn, qd * 4, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    std::memcpy(out, ctx->hstage, qd * 4);
     return 0;
 }
 
@@ -1933,8 +1983,9 @@ static int verify_alloc(fl_ctx *ctx) {
     ALLOC(ctx, ctx->vaq, M * qd);
     ALLOC(ctx, ctx->vas, M * (qd / 32) * 4);
     ALLOC(ctx, ctx->vasum, M * (qd / 32) * 4);
-    ALLOC(ctx, ctx->vtok, (size_t)kWideTokens * 4);
-    ALLOC(ctx, ctx->vpos, 4);
+    // the position, then (16 bytes on) the tokens: fl_verify copies both at once
+    ALLOC(ctx, ctx->vpos, 16 + (size_t)kWideTokens * 4);
+    ctx->vtok = ctx->vpos + 4;
     ALLOC(ctx, ctx->vslots, M * 8);
     ALLOC(ctx, ctx->vhq, M * F);
     ALLOC(ctx, ctx->vhs, M * (F / 32) * 4);
@@ -2210,7 +2261,7 @@ int fl_op_batched_matvec_f32in(fl_ctx *ctx, const fl_weight *w, int n_tokens, co
 }
 
 // The verify pass for M tokens at the device positions vpos.. (tokens in
-// vtok, vslots cleared); dev_pos: the cache writers read the position from the
+// vtok); dev_pos: the cache writers read the position from the
 // device too (graph capture), pos0 is then only used for planning checks.
 // What a pass of enqueue_verify produces: the greedy key of every token
 // (speculative verify), nothing (prefill chunks before the last), or the key
@@ -2230,7 +2281,8 @@ static int last_token_output(fl_ctx *ctx, const float *xt, int out_mode, unsigne
     const fl_weight &O = ctx->tied ? ctx->embed : ctx->output;
     const float eps = ctx->cfg.rms_norm_eps;
     const bool q8out = q8_output(ctx);
-    const int epi = out_mode == VOUT_LAST_LOGITS ? EPI_STORE : EPI_ARGMAX;
+    const int epi = out_mode == VOUT_LAST_LOGITS ? EPI_STORE_ARGMAX : EPI_ARGMAX;
+    if (out_mode == VOUT_LAST_LOGITS) slot = logits_key(ctx);  // cleared by the pass's embedding kernel
     if (O.format == FL_Q4K && !q8out) return fail(ctx, FL_E_UNSUPPORTED, "Q4_K output with Q8_0 layers");
     if (q8out)
         return launch_q8in(ctx, O, PRO_NORMQ1, epi, xt, ctx->out_norm, eps, nullptr, nullptr, nullptr, ctx->logits,
@@ -2247,7 +2299,9 @@ static int enqueue_verify(fl_ctx *ctx, int M, int pos0, bool dev_pos, int out_mo
     const int pro = ctx->layer_fmt == FL_Q8_0 ? PRO_NORMQ0 : PRO_NORMQ1;
     hipStream_t st = ctx->stream;
     float *xa = ctx->vx;
-    HIPCHK(ctx, launch_v_embed(ctx->embed.format, st, ctx->embed.desc(), ctx->vtok, M, xa));
+    const bool last_logits = out_mode == VOUT_LAST_LOGITS;
+    HIPCHK(ctx, launch_v_embed(ctx->embed.format, st, ctx->embed.desc(), ctx->vtok, M, xa,
+                               last_logits ? logits_key(ctx) : ctx->vslots, last_logits ? 1 : M));
     // Q4_K layers, up to 8 tokens: the QKV post and SiLU run inside the GEMMs
     const bool fuse = ctx->verify_fuse && ctx->layer_fmt == FL_Q4K && M <= 8 &&
                       std::max(qd + 2 * kvd, 2 * F) / 64 <= kVerifyCounters;
@@ -2449,12 +2503,11 @@ static int verify_check(fl_ctx *ctx, const uint32_t *tokens, int M, int pos0) {
 // One pass of M (<= kVerifyMaxTokens) tokens at pos0; the token ids are
 // already in ctx->vtok.  `*pos_host` must stay valid until the stream
 // reaches the pass (the position is copied to the device asynchronously).
-static int run_verify_pass(fl_ctx *ctx, int M, const int *pos_host, int out_mode) {
+static int run_verify_pass(fl_ctx *ctx, int M, const int *pos_host, int out_mode, bool pos_there = false) {
     const fl_model_config &c = ctx->cfg;
     hipStream_t st = ctx->stream;
     const int G = c.num_heads / c.num_kv_heads;
-    HIPCHK(ctx, hipMemcpyAsync(ctx->vpos, pos_host, 4, hipMemcpyHostToDevice, st));
-    if (out_mode != VOUT_NONE) HIPCHK(ctx, hipMemsetAsync(ctx->vslots, 0, (size_t)M * 8, st));
+    if (!pos_there) HIPCHK(ctx, hipMemcpyAsync(ctx->vpos, pos_host, 4, hipMemcpyHostToDevice, st));
     int rc = ensure_part(ctx, (size_t)M * c.num_kv_heads * part_splits(ctx) * G * (c.head_dim + 2));
     if (rc) return rc;
     // F32 / F16 / Q8 caches: one captured graph per (batch size, output
@@ -2504,12 +2557,16 @@ int fl_verify(fl_ctx *ctx, const uint32_t *tokens, int n_tokens, int pos0, int32
         return 0;
     }
     hipStream_t st = ctx->stream;
-    std::vector<int> tk(tokens, tokens + M);
-    HIPCHK(ctx, hipMemcpyAsync(ctx->vtok, tk.data(), (size_t)M * 4, hipMemcpyHostToDevice, st));
-    rc = run_verify_pass(ctx, M, &pos0, VOUT_ALL);
+    // position and tokens in one copy, the keys back in another (pinned; every
+    // call waits for the stream)
+    int *in = (int *)ctx->hstage;
+    in[0] = pos0;
+    for (int i = 0; i < M; i++) in[4 + i] = (int)tokens[i];
+    HIPCHK(ctx, hipMemcpyAsync(ctx->vpos, in, 16 + (size_t)M * 4, hipMemcpyHostToDevice, st));
+    rc = run_verify_pass(ctx, M, &pos0, VOUT_ALL, true);
     if (rc) return rc;
-    std::vector<unsigned long long> keys(M);
-    HIPCHK(ctx, hipMemcpyAsync(keys.data(), ctx->vslots, (size_t)M * 8, hipMemcpyDeviceToHost, st));
+    unsigned long long *keys = (unsigned long long *)(ctx->hstage + 256);
+    HIPCHK(ctx, hipMemcpyAsync(keys, ctx->vslots, (size_t)M * 8, hipMemcpyDeviceToHost, st));
     if (ctx->probe_layer >= 0 && ctx->probe_host)
         HIPCHK(ctx, hipMemcpyAsync(ctx->probe_host, ctx->probe_dev, ctx->probe_bytes, hipMemcpyDeviceToHost, st));
     HIPCHK(ctx, hipStreamSynchronize(st));
@@ -2601,7 +2658,9 @@ static int enqueue_wide(fl_ctx *ctx, int M, int pos0, int out_mode) {
     auto f32at = [&](size_t o) { return (float *)(ctx->wide + o); };
     float *x = f32at(B.x), *part = f32at(B.part);
     char *xp = ctx->wide + B.xp, *ap = ctx->wide + B.ap, *hp = ctx->wide + B.hp;
-    HIPCHK(ctx, launch_v_embed(ctx->embed.format, st, ctx->embed.desc(), ctx->vtok, M, x));
+    const bool last_logits = out_mode == VOUT_LAST_LOGITS;
+    HIPCHK(ctx, launch_v_embed(ctx->embed.format, st, ctx->embed.desc(), ctx->vtok, M, x,
+                               last_logits ? logits_key(ctx) : ctx->vslots, 1));
     int ks = 0;
     auto gemm = [&](const fl_weight &w, const char *in) {
         const BgPlan p = bgemm_plan(w.format, w.rows, w.cols, M);
@@ -2721,7 +2780,6 @@ int fl_prefill(fl_ctx *ctx, const uint32_t *tokens, int n_tokens, int pos0, floa
         const int mode = k + 1 < nchunks ? VOUT_NONE : out_logits ? VOUT_LAST_LOGITS : VOUT_LAST_ARGMAX;
         if (M > C) {
             HIPCHK(ctx, hipMemcpyAsync(ctx->vpos, &pos[k], 4, hipMemcpyHostToDevice, st));
-            if (mode != VOUT_NONE) HIPCHK(ctx, hipMemsetAsync(ctx->vslots, 0, 8, st));
             rc = enqueue_wide(ctx, M, pos[k], mode);
             slot = 0;
         } else {
@@ -2730,21 +2788,11 @@ int fl_prefill(fl_ctx *ctx, const uint32_t *tokens, int n_tokens, int pos0, floa
         }
         if (rc) return rc;
     }
+    if (out_logits) return read_logits(ctx, true, out_logits, out_token, out_val);
     unsigned long long key = 0;
     HIPCHK(ctx, hipMemcpyAsync(&key, ctx->vslots + slot, 8, hipMemcpyDeviceToHost, st));
-    if (out_logits)
-        HIPCHK(ctx, hipMemcpyAsync(out_logits, ctx->logits, (size_t)ctx->cfg.vocab_size * 4, hipMemcpyDeviceToHost, st));
     HIPCHK(ctx, hipStreamSynchronize(st));
-    if (out_logits) {
-        int bi = 0;
-        float bv = -INFINITY;
-        for (int i = 0; i < ctx->cfg.vocab_size; i++)
-            if (out_logits[i] > bv) { bv = out_logits[i]; bi = i; }
-        if (out_token) *out_token = bi;
-        if (out_val) *out_val = bv;
-    } else {
-        unpack_key(key, out_token, out_val);
-    }
+    unpack_key(key, out_token, out_val);
     return 0;
 }
 

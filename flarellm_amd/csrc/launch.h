@@ -193,7 +193,8 @@ hipError_t launch_b_silu(hipStream_t st, const float *part, int ksplit, int M, i
 
 // speculative verify (verify.hip)
 hipError_t launch_vgemm(int fmt, hipStream_t st, const VgArgs &a);
-hipError_t launch_v_embed(int fmt, hipStream_t st, const WDesc &E, const int *tokens, int M, float *x);
+hipError_t launch_v_embed(int fmt, hipStream_t st, const WDesc &E, const int *tokens, int M, float *x,
+                          unsigned long long *slots, int nslots);
 hipError_t launch_v_resnorm(int pro, hipStream_t st, const float *part, int ksplit, int M, int H, float *x,
                             const float *w, float eps, int8_t *q, float *s, int *sum);
 hipError_t launch_v_qkv_post(hipStream_t st, const float *part, int ksplit, int M, int rows,

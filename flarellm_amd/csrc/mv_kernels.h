@@ -7,7 +7,9 @@
 
 namespace fl {
 
-enum Epi { EPI_STORE = 0, EPI_ADD = 1, EPI_ARGMAX = 2, EPI_QKV = 3 };
+// EPI_STORE_ARGMAX: rows stored and their first maximum committed to the slot
+// as a scan of the stored row finds it (NaN and -inf never win; 0 = none)
+enum Epi { EPI_STORE = 0, EPI_ADD = 1, EPI_ARGMAX = 2, EPI_QKV = 3, EPI_STORE_ARGMAX = 4 };
 
 // EPI_QKV: the fused QKV matvec stores q (after RoPE) and writes the new
 // token's K (after RoPE) and V straight into the KV cache.  The weight rows
@@ -281,6 +283,17 @@ __device__ __forceinline__ unsigned long long rows_best(const float *acc, int ro
 #pragma unroll
     for (int r = 0; r < R; r++)
         if (row0 + r < rows) best = umax64(best, argmax_key(acc[r], (uint32_t)(row0 + r)));
+    return best;
+}
+
+// The same for EPI_STORE_ARGMAX: values above -inf only, -0 equal to 0.
+template <int R>
+__device__ __forceinline__ unsigned long long rows_best_scan(const float *acc, int row0, int rows) {
+    unsigned long long best = 0;
+#pragma unroll
+    for (int r = 0; r < R; r++)
+        if (row0 + r < rows && acc[r] > -INFINITY)
+            best = umax64(best, argmax_key(acc[r] + 0.0f, (uint32_t)(row0 + r)));
     return best;
 }
 

@@ -366,7 +366,7 @@ struct MvsArgs {
     const float *gs;
     const int *gsum;
     float *out;
-    unsigned long long *slot;  // EPI_ARGMAX
+    unsigned long long *slot;  // EPI_ARGMAX, EPI_STORE_ARGMAX
     QkvEpi qkv;                // EPI_QKV
     // gate/up: F hidden units, Q8_0 output blocks, optional f32 copy
     int F;
@@ -858,6 +858,9 @@ __device__ __forceinline__ void mvs_body(const MvsArgs &a, char *smem, int gw, i
             const int row0 = rg * R;
             if (a.epi == EPI_ARGMAX) {
                 best = umax64(best, rows_best<R>(acc, row0, W.rows));
+            } else if (a.epi == EPI_STORE_ARGMAX) {
+                best = umax64(best, rows_best_scan<R>(acc, row0, W.rows));
+                store_rows<R>(acc, row0, W.rows, lane, EPI_STORE, a.out);
             } else if (a.epi == EPI_ADD) {
                 // residual add (model.rs:2305-2311, 2537-2543): lane r adds row r
                 const float v = lane_row<R>(acc, lane);
@@ -876,7 +879,7 @@ __device__ __forceinline__ void mvs_body(const MvsArgs &a, char *smem, int gw, i
     // consumed
     pingpong(nunits, ta, tb, load, consume);
     MV_TS(4);
-    if (a.epi == EPI_ARGMAX) {
+    if (a.epi == EPI_ARGMAX || a.epi == EPI_STORE_ARGMAX) {
         float *red = (float *)(smem + mvs_lds_fmt<FMT, F32IN>(K) - 64 * 4 - (F32IN ? 0 : 64));
         wg_argmax_commit(best, a.slot, (unsigned long long *)red);
     }

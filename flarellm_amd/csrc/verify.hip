@@ -84,12 +84,13 @@ hipError_t launch_vgemm(int fmt, hipStream_t st, const VgArgs &a) {
     return hipGetLastError();
 }
 
-hipError_t launch_v_embed(int fmt, hipStream_t st, const WDesc &E, const int *tokens, int M, float *x) {
+hipError_t launch_v_embed(int fmt, hipStream_t st, const WDesc &E, const int *tokens, int M, float *x,
+                          unsigned long long *slots, int nslots) {
     switch (fmt) {
-    case F_Q8_0: hipLaunchKernelGGL(k_v_embed<F_Q8_0>, dim3(M), dim3(256), 0, st, E, tokens, x); break;
-    case F_Q6K: hipLaunchKernelGGL(k_v_embed<F_Q6K>, dim3(M), dim3(256), 0, st, E, tokens, x); break;
-    case F_Q4K: hipLaunchKernelGGL(k_v_embed<F_Q4K>, dim3(M), dim3(256), 0, st, E, tokens, x); break;
-    default: hipLaunchKernelGGL(k_v_embed<F_F32>, dim3(M), dim3(256), 0, st, E, tokens, x); break;
+    case F_Q8_0: hipLaunchKernelGGL(k_v_embed<F_Q8_0>, dim3(M), dim3(256), 0, st, E, tokens, x, slots, nslots); break;
+    case F_Q6K: hipLaunchKernelGGL(k_v_embed<F_Q6K>, dim3(M), dim3(256), 0, st, E, tokens, x, slots, nslots); break;
+    case F_Q4K: hipLaunchKernelGGL(k_v_embed<F_Q4K>, dim3(M), dim3(256), 0, st, E, tokens, x, slots, nslots); break;
+    default: hipLaunchKernelGGL(k_v_embed<F_F32>, dim3(M), dim3(256), 0, st, E, tokens, x, slots, nslots); break;
     }
     return hipGetLastError();
 }

@@ -930,10 +930,13 @@ __device__ __forceinline__ float4 vsum_part4(const float *part, int ksplit, int 
     return p;
 }
 
-// Embedding rows of the M tokens (token_embedding lookup, model.rs:1964).
+// Embedding rows of the M tokens (token_embedding lookup, model.rs:1964); also
+// clears the pass's argmax keys (slots[0 .. nslots)).
 template <int FMT>
-__global__ __launch_bounds__(256) void k_v_embed(WDesc E, const int *tokens, float *x) {
+__global__ __launch_bounds__(256) void k_v_embed(WDesc E, const int *tokens, float *x, unsigned long long *slots,
+                                                 int nslots) {
     const int t = blockIdx.x, H = E.cols;
+    if (threadIdx.x == 0 && t < nslots) slots[t] = 0ull;
     const int row = min(max(tokens[t], 0), E.rows - 1);
     for (int i = threadIdx.x; i < H; i += blockDim.x) {
         float v;
