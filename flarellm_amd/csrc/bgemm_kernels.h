@@ -230,13 +230,17 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     const int row0 = (rt * NW + wave) * 32;
     const size_t row = min(row0 + l31, W.rows - 1);
 
+    const uint32_t lane16 = lane * 16;
     auto stage = [&](int buf, int st) {
 #pragma unroll
         for (int c = 0; c < (TT * RC + NW - 1) / NW; c++) {
             const int p = wave + c * NW, tt = p / RC, kb = p % RC;
             if ((c + 1) * NW > TT * RC && p >= TT * RC) break;  // the last round may be partial
-            const char *src = a.xp + ((size_t)min(tile0 + tt, ntile - 1) * a.nst + st) * kPackRec + kb * 1024;
-            copy_to_lds(src + lane * 16, smem + (buf * TT + tt) * kPackRec + kb * 1024);
+            // 32-bit scalar offset (packed activations are below 4 GiB): the
+            // lanes' part of the address is then one register for all copies
+            uint32_t off = (uint32_t)(min(tile0 + tt, ntile - 1) * a.nst + st) * kPackRec + kb * 1024;
+            asm("" : "+s"(off));
+            copy_to_lds(a.xp + off + lane16, smem + (buf * TT + tt) * kPackRec + kb * 1024);
         }
     };
 
@@ -250,60 +254,86 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     if constexpr (FMT == F_Q4K) {
         float *dl = (float *)(smem + 2 * TT * kPackRec) + wave * 32;  // d of the wave's rows
         const uint8_t *qp = W.q + row * a.nst * 128 + 16 * h, *hp = W.h + row * a.nst * 16;
-        u4x_t wn[4], hn;
-        auto wload = [&](int st) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) wn[j] = *(const u4x_t *)(qp + (size_t)st * 128 + 32 * j);
-            hn = *(const u4x_t *)(hp + (size_t)st * 16);
-        };
+        // Weights: one step in registers; a piece is loaded again for the next
+        // step as soon as its codes are unpacked.
+        u4x_t w[4], hd;
+        auto wload = [&](int st, int j) { w[j] = *(const u4x_t *)(qp + (size_t)st * 128 + 32 * j); };
         stage(0, s0);
-        wload(s0);
+        asm volatile("" ::: "memory");  // the copies first: the wait below counts the loads after them
+#pragma unroll
+        for (int j = 0; j < 4; j++) wload(s0, j);
+        hd = *(const u4x_t *)(hp + (size_t)s0 * 16);
         for (int st = s0; st < s1; st++) {
-            const int cur = (st - s0) & 1;
-            const u4x_t w[4] = {wn[0], wn[1], wn[2], wn[3]}, hd = hn;
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's copies have landed
-            __syncthreads();
-            const int nx = min(st + 1, s1 - 1);
+            const int cur = (st - s0) & 1, nx = min(st + 1, s1 - 1);
+            // this wave's copies have landed (loads complete in order, and the
+            // five weight loads issued after them may be in flight) and its
+            // reads of the other buffer are complete
+            asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
             if (st + 1 < s1) stage(cur ^ 1, nx);
-            wload(nx);
+            asm volatile("" ::: "memory");
             const char *buf = smem + cur * TT * kPackRec;
             // unpack_q4k_scales (model.rs:8709-8719), flare packing
             const uint32_t sa = hd[1], sb = hd[2], sc = hd[3];
             if (h == 0) dl[l31] = h2f((uint16_t)(hd[0] & 0xFFFF));
-            f16x_t C[TT];
+            // Blocks in the order 0 4 1 5 2 6 3 7 (two share their bytes), TT
+            // token tiles each: unit i = (block i / TT, tile i % TT).  The
+            // multiply-adds of unit i - 1 are issued between the two MFMAs of
+            // unit i and after them, so the matrix and the vector units of the
+            // SIMD work at once (in the order the compiler chose, each unit's
+            // MFMAs, a wait, then its multiply-adds, two 8B-shaped layers and
+            // 4096 tokens took 7.85 ms against 7.1).  What bounds it then is
+            // vector issue: ~1000 instructions and 76 MFMAs per wave and step,
+            // two waves per SIMD, fill ~90 % of its slots.
+            f16x_t C[TT], dd[2];
+            h8x_t A[2], B[2][2];
+            float s3[3];
+            auto unpack = [&](int bi, int half) {  // half of block bi's weight operand
+                const int j = bi >> 1, hi = bi & 1;
+                const uint32_t s8 = (sa >> (8 * j)) & 0xFF;
+                const uint32_t six = hi ? (s8 >> 6) | (((sc >> (8 * j)) & 0xF) << 2) : s8 & 63;
+                const float fs = (float)six;
+                const h2x_t mul = h2_both(fs), add = h2_both(fs * -72.0f);
+                uint32_t o[4];
+                if (hi) q4_pairs<false>(w[j][2 * half], w[j][2 * half + 1], mul, add, o);
+                else q4_pairs<true>(w[j][2 * half], w[j][2 * half + 1], mul, add, o);
+                A[half] = as_h8(u4x_t{o[0], o[1], o[2], o[3]});
+                if (hi && half) wload(nx, j);
+            };
+            auto fetch = [&](int i) {  // unit i's activations
+                const int bi = i / TT, blk = (bi >> 1) + 4 * (bi & 1);
+                const char *rec = buf + (i % TT) * kPackRec;
+                B[i & 1][0] = *(const h8x_t *)(rec + blk * 2048 + lane * 16);
+                B[i & 1][1] = *(const h8x_t *)(rec + blk * 2048 + 1024 + lane * 16);
+                s3[i % 3] = *(const float *)(rec + kPackScale + blk * 128 + l31 * 4);
+            };
+            auto madd = [&](int i, int half) {  // half of unit i's multiply-adds
+                const int tt = i % TT;
+                const float sv = s3[i % 3];
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
+                for (int e = 8 * half; e < 8 * half + 8; e++)
+                    C[tt][e] = i < TT ? sv * dd[i & 1][e] : __builtin_fmaf(sv, dd[i & 1][e], C[tt][e]);
+            };
+            unpack(0, 0);
+            unpack(0, 1);
+            fetch(0);
 #pragma unroll
-                for (int hi = 0; hi < 2; hi++) {
-                    const int blk = j + 4 * hi;
-                    const uint32_t s8 = (sa >> (8 * j)) & 0xFF;
-                    const uint32_t six = hi ? (s8 >> 6) | (((sc >> (8 * j)) & 0xF) << 2) : s8 & 63;
-                    const float fs = (float)six;
-                    const h2x_t mul = h2_both(fs), add = h2_both(fs * -72.0f);
-                    uint32_t o0[4], o1[4];
-                    if (hi) {
-                        q4_pairs<false>(w[j][0], w[j][1], mul, add, o0);
-                        q4_pairs<false>(w[j][2], w[j][3], mul, add, o1);
-                    } else {
-                        q4_pairs<true>(w[j][0], w[j][1], mul, add, o0);
-                        q4_pairs<true>(w[j][2], w[j][3], mul, add, o1);
-                    }
-                    const h8x_t a0 = as_h8(u4x_t{o0[0], o0[1], o0[2], o0[3]});
-                    const h8x_t a1 = as_h8(u4x_t{o1[0], o1[1], o1[2], o1[3]});
-#pragma unroll
-                    for (int tt = 0; tt < TT; tt++) {
-                        const char *rec = buf + tt * kPackRec;
-                        const h8x_t b0 = *(const h8x_t *)(rec + blk * 2048 + lane * 16);
-                        const h8x_t b1 = *(const h8x_t *)(rec + blk * 2048 + 1024 + lane * 16);
-                        const float s = *(const float *)(rec + kPackScale + blk * 128 + l31 * 4);
-                        f16x_t dd = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, b0, zero, 0, 0, 0);
-                        dd = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, b1, dd, 0, 0, 0);
-#pragma unroll
-                        for (int i = 0; i < 16; i++)
-                            C[tt][i] = blk == 0 ? s * dd[i] : __builtin_fmaf(s, dd[i], C[tt][i]);
-                    }
-                }
+            for (int i = 0; i < 8 * TT; i++) {
+                const int bi = i / TT, tt = i % TT;
+                __builtin_amdgcn_sched_barrier(0);
+                dd[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[0], B[i & 1][0], zero, 0, 0, 0);
+                if (i + 1 < 8 * TT) fetch(i + 1);
+                if (i > 0) madd(i - 1, 0);
+                if (bi < 7 && tt == TT - 1) unpack(bi + 1, 0);  // its operand has just been read
+                __builtin_amdgcn_sched_barrier(0);
+                dd[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[1], B[i & 1][1], dd[i & 1], 0, 0, 0);
+                if (i > 0) madd(i - 1, 1);
+                if (bi < 7 && tt == TT - 1) unpack(bi + 1, 1);
             }
+            __builtin_amdgcn_sched_barrier(0);
+            madd(8 * TT - 1, 0);
+            madd(8 * TT - 1, 1);
             // acc += d * C + sum_j c_j (s sum q)_j, c_j = 8 d sc_j - dmin mn_j
             // (C holds codes less 8): c_j and s sum q as three bfloat16 parts
             // each, the products of parts down to 2^-24 summed by the MFMA
@@ -328,11 +358,13 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
                 for (int k = 0; k < 3; k++) cp[k][p] = __builtin_amdgcn_perm(part[1][k], part[0][k], 0x07060302u);
             }
+            hd = *(const u4x_t *)(hp + (size_t)nx * 16);
             const b8x_t c1 = __builtin_bit_cast(b8x_t, u4x_t{cp[0][0], cp[0][1], cp[0][2], cp[0][3]});
             const b8x_t c2 = __builtin_bit_cast(b8x_t, u4x_t{cp[1][0], cp[1][1], cp[1][2], cp[1][3]});
+            const uint32_t hmask = 0u - (uint32_t)h;  // (a select here went through memory)
             u4x_t c13;
 #pragma unroll
-            for (int k = 0; k < 4; k++) c13[k] = h ? cp[2][k] : cp[0][k];
+            for (int k = 0; k < 4; k++) c13[k] = (cp[2][k] & hmask) | (cp[0][k] & ~hmask);
             const b8x_t c3 = __builtin_bit_cast(b8x_t, c13);
 #pragma unroll
             for (int tt = 0; tt < TT; tt++) {
