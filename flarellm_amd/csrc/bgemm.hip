@@ -78,6 +78,7 @@ hipError_t launch_bgemm(int fmt, hipStream_t st, const WDesc &W, const char *xp,
     a.part = part;
     a.nrt = p.nrt;
     a.ntt = p.ntt;
+    if (pack_bytes(M, W.cols) >> 32) return hipErrorInvalidValue;  // 32-bit offsets
     // every row, token and step belongs to a workgroup, every split has steps
     if ((long long)p.nrt * p.nw * 32 < W.rows || (long long)p.ntt * p.tt * kPackTile < M ||
         (long long)p.ksplit * p.chunk < a.nst || (long long)(p.ksplit - 1) * p.chunk >= a.nst)

@@ -66,3 +66,26 @@ def test_key_skips_what_is_not_a_number(backend):
         backend.upload_weights_to_gpu(model)
         logits, t, v = _step(backend, 9, 0)
         assert np.isnan(logits).any() and (t, v) == _scan(logits), case
+
+
+def test_replayed_logits_steps_match_the_first(backend):
+    """Steps with logits replay a graph from the second call on: every replay
+    against the same step enqueued directly (FL_OPT_EXACT off and on drops the
+    graph), with other work and synchronizations between."""
+    from flarellm_amd import _lib as L
+
+    spec = S.tiny_spec(FL_Q8_0, vocab=700)
+    backend.init_gpu_kv_cache(spec, FL_KV_F16)
+    backend.upload_weights_to_gpu(S.make_model(spec, seed=6))
+    toks = S.random_tokens(8, 12, spec.vocab).tolist()
+    want = []
+    for pos, t in enumerate(toks):
+        backend.set_option(L.FL_OPT_EXACT, 1)
+        backend.set_option(L.FL_OPT_EXACT, 0)  # drops captured graphs: this step is enqueued
+        want.append(_step(backend, t, pos))
+    backend.reset()
+    for pos, t in enumerate(toks):
+        logits, tok, val = _step(backend, t, pos)
+        assert np.array_equal(logits.view(np.uint32), want[pos][0].view(np.uint32)) and (tok, val) == want[pos][1:]
+        backend.forward_greedy(t, pos)  # the greedy step's own graph, same slot
+        backend.sync()
