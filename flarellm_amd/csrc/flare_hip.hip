@@ -2802,8 +2802,12 @@ int fl_prefill(fl_ctx *ctx, const uint32_t *tokens, int n_tokens, int pos0, floa
     static const int C = measure_env("FLARE_PREFILL_TOKENS")
                              ? std::max(1, std::min(kPrefillTokens, atoi(measure_env("FLARE_PREFILL_TOKENS"))))
                              : kPrefillTokens;
-    // prompts of more than one short pass: wide passes of up to kWideTokens
-    const bool wide = n_tokens > C && wide_possible(ctx) && wide_alloc(ctx, std::min(n_tokens, kWideTokens));
+    // wide passes of up to kWideTokens: of Q4_K layers from 17 tokens on (two
+    // 8B-shaped layers, 64 tokens 325 us against 361 in a short pass), of Q8_0
+    // layers where one short pass does not do (1B-shaped, 64 tokens 229 against
+    // 215 us; 65 tokens 260)
+    const int least = ctx->layer_fmt == FL_Q4K ? std::min(C, kVerifyMaxTokens) : C;
+    const bool wide = n_tokens > least && wide_possible(ctx) && wide_alloc(ctx, std::min(n_tokens, kWideTokens));
     const int step = wide ? ctx->wide_cap : C;
     const int nchunks = (n_tokens + step - 1) / step;
     // host copies stay alive until the final synchronisation
@@ -2814,7 +2818,7 @@ int fl_prefill(fl_ctx *ctx, const uint32_t *tokens, int n_tokens, int pos0, floa
         pos[k] = pos0 + t0;
         HIPCHK(ctx, hipMemcpyAsync(ctx->vtok, tk.data() + t0, (size_t)M * 4, hipMemcpyHostToDevice, st));
         const int mode = k + 1 < nchunks ? VOUT_NONE : out_logits ? VOUT_LAST_LOGITS : VOUT_LAST_ARGMAX;
-        if (M > C) {
+        if (wide && M > least) {
             HIPCHK(ctx, hipMemcpyAsync(ctx->vpos, &pos[k], 4, hipMemcpyHostToDevice, st));
             rc = enqueue_wide(ctx, M, pos[k], mode);
             slot = 0;
