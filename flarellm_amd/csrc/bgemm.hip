@@ -30,17 +30,32 @@ hipError_t launch_tt(int tt, hipStream_t st, const BgArgs &a) {
 
 }  // namespace
 
-// The plan of least estimated time.  A workgroup of 8 waves (or two of 4
-// waves with at most 2 token tiles) fills a CU; measured per 256-value step
-// and round of the chip on MI355X (28672 x 4096 Q4_K, 2048 tokens): 2.9, 4.3,
-// 5.4 and 7.0 us with 1, 2, 3 and 4 token tiles.  K is split where tiles alone
-// leave CUs idle; the split's partial sums cost a write, a read (4 TB/s
-// together) and a launch.  Q8_0 sums every 32-block straight into its output,
-// so a split holds at most kQ8Steps steps (7168 values: 1.4e-7 against 64 bits
-// where 14336 in one chain had 2.0e-7).
+// The plan of least estimated time.  A workgroup of 8 waves, or two of 4 waves
+// with at most 2 token tiles, fills a CU.  The costs are a least-squares fit to
+// the times of all plans of 14 shapes on MI355X (576 x 576 to 14336 x 4096 and
+// 4096 x 14336, 32 to 2048 tokens; 6 to 7 % mean error): per 256-value step,
+// per round of the chip, and per MB of partial sums written; two workgroups of
+// 4 waves are priced 10 % above the fit, which let them take near ties that
+// they lose.  Split sums also cost their read (4 TB/s) and, unless the kernel
+// behind sums them in any case (summed), a launch of 4 us.  Over those shapes
+// and 15 others the plan taken is 1 to 2 % above the best; one cost per step
+// for both formats and wave counts was 8 to 9 % above (4096 x 4096 Q4_K, 509
+// tokens: 52 us unsplit where 33 are reached).
+// Q8_0 sums every 32-block straight into its output, so a split holds at most
+// kQ8Steps steps (7168 values: 1.4e-7 against 64 bits where 14336 in one chain
+// had 2.0e-7).
 constexpr int kQ8Steps = 28;
-BgPlan bgemm_plan(int fmt, int rows, int cols, int M) {
-    static const double step_us[5] = {0, 2.9, 4.3, 5.4, 7.0};
+struct BgCost {
+    double step8[4];  // 8 waves: us per step with 1..4 token tiles
+    double step4[2];  // 4 waves, two workgroups on a CU
+    double alone[2];  // 4 waves, one on a CU
+    double round, mb;
+};
+constexpr BgCost kCostQ8{{3.61, 4.27, 5.32, 6.71}, {3.34, 4.35}, {2.30, 3.21}, 2.3, 0.165};
+constexpr BgCost kCostQ4{{2.53, 3.52, 4.57, 5.81}, {2.43, 3.63}, {1.72, 2.53}, 1.6, 0.126};
+BgPlan bgemm_plan(int fmt, int rows, int cols, int M, bool summed) {
+    const BgCost &c = fmt == F_Q8_0 ? kCostQ8 : kCostQ4;
+    const double mb = (double)M * rows * 4 / 1e6;
     const int tiles = (M + kPackTile - 1) / kPackTile, nst = (cols + 255) / 256;
     BgPlan best{};
     double best_us = 0;
@@ -56,8 +71,9 @@ BgPlan bgemm_plan(int fmt, int rows, int cols, int M) {
                 p.ksplit = (nst + p.chunk - 1) / p.chunk;
                 if (p.ksplit != want || (fmt == F_Q8_0 && p.chunk > kQ8Steps)) continue;
                 const long long wgs = (long long)p.nrt * p.ntt * p.ksplit, slots = nw == 8 ? 256 : 512;
-                double us = (double)((wgs + slots - 1) / slots) * p.chunk * step_us[tt];
-                if (p.ksplit > 1) us += 4.0 + 2.0 * p.ksplit * M * (double)rows * 4 / 4e6;
+                const double step = nw == 8 ? c.step8[tt - 1] : wgs <= 256 ? c.alone[tt - 1] : c.step4[tt - 1];
+                double us = (double)((wgs + slots - 1) / slots) * (p.chunk * step + c.round) + p.ksplit * mb * c.mb;
+                if (p.ksplit > 1) us += summed ? (p.ksplit - 1) * mb / 4 : 4.0 + p.ksplit * mb / 4;
                 if (!best.tt || us < best_us) {
                     best = p;
                     best_us = us;

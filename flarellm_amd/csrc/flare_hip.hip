@@ -2198,7 +2198,7 @@ int fl_op_batched_dequant_matmul(fl_ctx *ctx, const fl_weight *w, const float *i
         // then one GEMM per kBatchRows rows
         for (int b0 = 0; b0 < batch && e == hipSuccess; b0 += kBatchRows) {
             const int n = std::min(kBatchRows, batch - b0);
-            const BgPlan p = bgemm_plan(w->format, w->rows, cols, n);
+            const BgPlan p = bgemm_plan(w->format, w->rows, cols, n, false);
             const size_t xb = pack_bytes(n, cols);
             const int rc = ws_ensure(ctx, xb + (p.ksplit > 1 ? (size_t)p.ksplit * n * w->rows * 4 : 0));
             if (rc) return rc;
@@ -2632,7 +2632,7 @@ static WideBufs wide_layout(const fl_ctx *ctx, int cap) {
     const size_t shapes[4][2] = {{qd + 2 * kvd, H}, {H, qd}, {2 * F, H}, {H, F}};
     for (const auto &s : shapes)
         for (int m = 1; m <= cap; m++)
-            part = std::max(part, (size_t)bgemm_plan(ctx->layer_fmt, (int)s[0], (int)s[1], m).ksplit * m * s[0]);
+            part = std::max(part, (size_t)bgemm_plan(ctx->layer_fmt, (int)s[0], (int)s[1], m, true).ksplit * m * s[0]);
     b.x = take(M * H * 4);
     b.q = take(M * qd * 4);
     b.planes = ctx->kv_format == FL_KV_F32 || ctx->kv_format == FL_KV_Q8;
@@ -2699,7 +2699,7 @@ static int enqueue_wide(fl_ctx *ctx, int M, int pos0, int out_mode) {
                                last_logits ? logits_key(ctx) : ctx->vslots, 1));
     int ks = 0;
     auto gemm = [&](const fl_weight &w, const char *in) {
-        const BgPlan p = bgemm_plan(w.format, w.rows, w.cols, M);
+        const BgPlan p = bgemm_plan(w.format, w.rows, w.cols, M, true);
         ks = p.ksplit;
         return launch_bgemm(w.format, st, w.desc(), in, M, p, part);
     };

@@ -178,12 +178,13 @@ struct MvoArgs;
 hipError_t launch_mvo(int fmt, hipStream_t st, const MvoArgs &a);
 
 // large-batch GEMM (bgemm.hip): workgroup tiles of 32 nw rows x 32 tt tokens,
-// K in ksplit chunks of 256-value steps
+// K in ksplit chunks of 256-value steps; summed: the kernel that reads the
+// result takes any number of partial sums
 constexpr int kBgMaxSplit = 32;
 struct BgPlan {
     int tt, nw, nrt, ntt, ksplit, chunk;
 };
-BgPlan bgemm_plan(int fmt, int rows, int cols, int M);
+BgPlan bgemm_plan(int fmt, int rows, int cols, int M, bool summed);
 hipError_t launch_bgemm(int fmt, hipStream_t st, const WDesc &W, const char *xp, int M, const BgPlan &p, float *part);
 hipError_t launch_quant_pack(hipStream_t st, const float *x, int M, int K, char *xp);
 hipError_t launch_b_resnorm(int pro, hipStream_t st, const float *part, int ksplit, int M, int H, float *x,
