@@ -371,7 +371,7 @@ def run_decode(args, config: str, with_cpu: bool) -> dict:
                 "kernel": f"{dom} ({d['kernel']})", "bytes_per_launch": d["bytes"],
                 "avg_launch_us": d["us"]}
 
-    # time to first token through fl_prefill (64-token int8-MFMA passes) of
+    # time to first token through fl_prefill (passes of up to 2048 tokens) of
     # the same prompt, against the decode-step path above
     prefill = None
     if n_prompt > 1:
@@ -388,7 +388,7 @@ def run_decode(args, config: str, with_cpu: bool) -> dict:
         plg, _, _ = b.forward_prefill(prompt, logits=True)
         top2 = np.sort(plg)[-2:]
         prefill = {"tokens": n_prompt, "ms": round(pms, 2), "tok_s": round(n_prompt * 1000.0 / pms, 1),
-                   "pass_tokens": 64, "first_token": ptok, "decode_path_first_token": int(toks[0]),
+                   "pass_tokens": min(n_prompt, 2048), "first_token": ptok, "decode_path_first_token": int(toks[0]),
                    "top2_gap_rel": round(float((top2[1] - top2[0]) / abs(top2[1])), 5),
                    "decode_path_token_rank": int((plg > plg[int(toks[0])]).sum())}
         log(f"[bench {config}] prefill of {n_prompt} tokens: {pms:.2f} ms ({n_prompt * 1000.0 / pms:.0f} tok/s); "

@@ -200,7 +200,10 @@ __global__ __launch_bounds__(256) void k_b_residual_row(const float *part, int k
 // of 256 values.  Weights go from memory to registers (every row belongs to
 // one wave; the next step's are in flight), activations through a
 // double-buffered LDS slot that all waves share, copied there without
-// registers while the step before is consumed.
+// registers while the step before is consumed.  Bound by vector issue (the
+// multiply-adds of the block scales, the unpacking, the MFMAs' own issue), not
+// by memory.  Measured on MI355X: 14336 x 4096 Q4_K, 1000 rows 188 us (624
+// TFLOP/s; the call 4100 -> 213 us against 16 rows a launch).
 template <int FMT, int TT, int NW>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_bgemm(BgArgs a) {
     extern __shared__ __align__(16) char smem[];  // [2][TT][kPackRec], then [NW][32] floats

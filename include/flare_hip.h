@@ -188,7 +188,8 @@ int fl_op_batched_matvec_q8in(fl_ctx *ctx, const fl_weight *w, int n_tokens, con
  * (model.rs:468; CPU semantics model.rs:740-1036): input [batch][cols] f32
  * rows (device), each quantized on the device with quantize_input_q8_0_into,
  * then the quantized matvec of every row: out [batch][rows] (device).  Q8_0 /
- * Q4_K weights; any batch (16 rows per int8-MFMA GEMM).  Synchronises. */
+ * Q4_K weights; any batch (up to 16 rows on the int8-MFMA verify GEMM, more
+ * on the large-batch f16-MFMA GEMM, at most 2048 at once).  Synchronises. */
 int fl_op_batched_dequant_matmul(fl_ctx *ctx, const fl_weight *w, const float *input, int batch,
                                  float *out);
 /* ComputeBackend::prefill_attention_gpu (model.rs:336-368; softcap 0):
@@ -319,9 +320,11 @@ int fl_verify(fl_ctx *ctx, const uint32_t *tokens, int n_tokens, int pos0, int32
               float *out_vals);
 
 /* Model::forward_prefill (model.rs:2578-3040): n_tokens prompt tokens at
- * positions pos0..pos0+n_tokens-1 in batched passes of up to 16 tokens (the
- * fl_verify pass: int8-MFMA projections, causal attention over the cache
- * and the tokens before each one in the batch, K/V written to the cache),
+ * positions pos0..pos0+n_tokens-1 in batched passes: short ones of up to 64
+ * tokens (the fl_verify pass) and, from 65 tokens on (17 over Q4_K layers),
+ * wide ones of up to 2048 where device memory allows (exact block dots on f16
+ * MFMA, causal attention over the cache and the tokens before each one in the
+ * batch, K/V written to the cache),
  * then the output projection of the last token only.  The reference starts
  * from an empty cache (pos0 = 0); pos0 > 0 continues a cache whose slots
  * 0..pos0-1 are written.  out_logits (vocab_size host floats) may be NULL:
