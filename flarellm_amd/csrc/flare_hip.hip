@@ -1773,9 +1773,10 @@ static int decode_step(fl_ctx *ctx, uint32_t token, const float *embedding, int 
         // so the pinned words are free to write.
         ctx->hstep[0] = tok;
         ctx->hstep[1] = pos;
-        // Steps with logits replay a graph from their second call on (30 small
-        // layers, 152 launches: 717 -> 650 us a step); capturing on the first
-        // would make that one pay for it.
+        // Steps with logits replay a graph from their second call on: 4 layers
+        // of 1B widths 234 -> 226 us, 2 of 8B 240 -> 236; 30 small layers (152
+        // launches) 694-713 us against 697-769, by how fast the host enqueues.
+        // Capturing on the first would make that one pay for it.
         const bool graph = use_graph() && out_logits && !embedding && ctx->probe_layer < 0 && !ctx->exact;
         if (graph && !ctx->lgexec && ctx->logit_steps++ > 0) {
             const int rc = capture_logits_step(ctx);
