@@ -66,6 +66,15 @@ __device__ __forceinline__ void attw_split(const float *x, u4x_t *o) {
     }
 }
 
+// 16-bit operand values (binary16, or bfloat16 planes)
+template <int NP>
+constexpr uint32_t kAttwExp = NP == 1 ? 0x7C00u : 0x7F80u;  // exponent of Inf and NaN
+template <int NP>
+__device__ __forceinline__ float attw_value(uint16_t b) {
+    if constexpr (NP == 1) return h2f(b);
+    else return __uint_as_float((uint32_t)b << 16);
+}
+
 // the other half's value (lane ^ 32)
 __device__ __forceinline__ float attw_other(float v) { return __shfl_xor(v, 32, 64); }
 
@@ -78,15 +87,28 @@ __device__ __forceinline__ float attw_other(float v) { return __shfl_xor(v, 32, 
 // workgroup's chain of key tiles.  Measured on MI355X: 1531 f32 queries of 32
 // heads x 128: the call, split into planes included, 4180 -> 172
 // us against one query at a time on the vector units.
-template <int NP, int D>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_attw(AttwArgs a) {
+//
+// Values that are not finite: a masked key has p = 0, but its V row is in the
+// PV operand, and 0 * Inf is NaN; an Inf against the zero low part of p or q is
+// NaN where the product is Inf.  Every such case leaves a NaN or Inf in O, so
+// the workgroup looks at its O once, at the end (1531 queries as above: 172.2
+// us without, 170.8 with it), and if
+// one is there does its work again with CAREFUL: values of V that are not
+// finite are taken out of the operand and added for the queries that see them,
+// and scores that came out NaN are formed again in plain f32.  Every other
+// output is the same bits with and without CAREFUL.
+// Returns whether that is needed (the same for the whole workgroup).
+template <int NP, int D, bool CAREFUL>
+__device__ __forceinline__ bool attw_body(const AttwArgs &a) {
     constexpr int QP = NP == 1 ? 2 : 3;  // parts of q and p
     constexpr int KS = D / 16, DT = D / 32, CH = D / 8;  // K = 16 steps, channel tiles, 16-B chunks per row
     constexpr int PLANE = 64 * D * 2, BUF = NP * PLANE;  // bytes of 64 keys
     constexpr int NL = BUF / 1024 / 8;                   // copies per wave and tile
     extern __shared__ __align__(16) char smem[];         // 3 buffers; at the end the lanes' exchange
-    const int lane = threadIdx.x & 63, l31 = lane & 31, h = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = wave >> 2;
+    int tid = threadIdx.x;
+    if constexpr (CAREFUL) asm volatile("" : "+v"(tid));  // nothing of it is kept in registers through the first pass
+    const int lane = tid & 63, l31 = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), b = wave >> 2;
     const int kvh = blockIdx.x % a.nkv;
     const int ntile = (a.M + 31) / 32, items = ntile * a.group;
     const int w = (items + 3) / 4 - 1 - blockIdx.x / a.nkv;  // longest rows first
@@ -129,9 +151,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // otherwise go subnormal for small q)
     u4x_t qf[KS][QP];
     float c = (float)(1.4426950408889634 / (D == 64 ? 8.0 : 11.313708498984761));  // log2(e) * the score scale
+    float qmul = 1.0f;
     {
         const float *qp = a.q + (size_t)min(t, a.M - 1) * a.qstride + head * D + 8 * h;
-        float mul = 1.0f;
         if constexpr (NP == 1) {
             float m = 0.0f;
 #pragma unroll
@@ -143,7 +165,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const int e = (int)((__float_as_uint(m) >> 23) & 0xFF);
             if (e > 13 && e < 255) {
                 const int s = min(max(140 - e, -100), 100);
-                mul = __uint_as_float((uint32_t)(127 + s) << 23);
+                qmul = __uint_as_float((uint32_t)(127 + s) << 23);
                 c *= __uint_as_float((uint32_t)(127 - s) << 23);
             }
         }
@@ -151,7 +173,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int k = 0; k < KS; k++) {
             float x[8];
 #pragma unroll
-            for (int j = 0; j < 8; j++) x[j] = qp[16 * k + j] * mul;
+            for (int j = 0; j < 8; j++) x[j] = qp[16 * k + j] * qmul;
             attw_split<NP>(x, qf[k]);
         }
     }
@@ -202,6 +224,31 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 for (int i = 0; i < 16; i++)
                     if (kb + 16 * (i >> 3) + 8 * h + (i & 7) > qpos) s[i] = -INFINITY;
             }
+            if constexpr (CAREFUL) {
+                // (one score at a time, indexed by selects: registers matter here, time does not)
+                const float *qp = a.q + (size_t)min(t, a.M - 1) * a.qstride + head * D;
+                const char *k0 = smem + bk * BUF + 32 * b * D * 2;
+#pragma unroll 1
+                for (int i = 0; i < 16; i++) {
+                    float v = s[0];
+#pragma unroll
+                    for (int j = 1; j < 16; j++) v = i == j ? s[j] : v;
+                    if (v == v) continue;
+                    const int key = 16 * (i >> 3) + 8 * h + (i & 7), g = (key & 3) | ((key >> 1) & 4);
+                    v = 0.0f;
+#pragma unroll 1
+                    for (int d = 0; d < D; d++) {
+                        const char *kp = k0 + key * D * 2 + (((d >> 3) ^ g) * 16) + (d & 7) * 2;
+                        float kv = attw_value<NP>(*(const uint16_t *)kp);
+                        if constexpr (NP == 3)
+                            kv += attw_value<NP>(*(const uint16_t *)(kp + PLANE)) +
+                                  attw_value<NP>(*(const uint16_t *)(kp + 2 * PLANE));
+                        v = __builtin_fmaf(qp[d] * qmul, kv, v);
+                    }
+#pragma unroll
+                    for (int j = 0; j < 16; j++) s[j] = i == j ? v : s[j];
+                }
+            }
             float m = s[0];
 #pragma unroll
             for (int i = 1; i < 16; i++) m = fmaxf(m, s[i]);
@@ -249,6 +296,21 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
                     for (int p = 0; p < NP; p++)
                         vf[mm][p] = *(const u4x_t *)(vt + p * PLANE + dd * 64 + (((2 * mm + h) ^ ((dd >> 1) & 3)) * 16));
+                uint32_t bad = 0;  // CAREFUL: keys of the tile whose V row is not finite in these channels
+                if constexpr (CAREFUL) {
+                    constexpr uint32_t E = kAttwExp<NP>;
+#pragma unroll
+                    for (int mm = 0; mm < 2; mm++)
+#pragma unroll
+                        for (int j = 0; j < 8; j++) {
+                            const uint32_t w = vf[mm][0][j >> 1], sh = 16 * (j & 1);
+                            if (((w >> sh) & E) != E) continue;
+                            vf[mm][0][j >> 1] = w & ~(0xFFFFu << sh);
+                            bad |= 1u << (16 * mm + 8 * h + j);
+                        }
+#pragma unroll
+                    for (int x = 1; x < 64; x <<= 1) bad |= __shfl_xor(bad, x, 64);
+                }
                 f16x_t pv = zero;
 #pragma unroll
                 for (int mm = 0; mm < 2; mm++) {
@@ -264,6 +326,25 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 for (int mm = 0; mm < 2; mm++) pv = attw_mfma<NP>(vf[mm][0], pf[mm][0], pv);
 #pragma unroll
                 for (int i = 0; i < 16; i++) o[d][i] = __builtin_fmaf(o[d][i], al, pv[i]);
+                if constexpr (CAREFUL) {
+                    for (; bad; bad &= bad - 1) {  // uniform
+                        const int key = __builtin_ctz(bad);
+                        float p = s[0];
+#pragma unroll
+                        for (int i = 1; i < 16; i++) p = i == (((key >> 4) << 3) | (key & 7)) ? s[i] : p;
+                        p = __shfl(p, l31 + 32 * ((key >> 3) & 1), 64);
+                        if (kb + key > qpos) continue;
+                        int h4 = 4 * h;
+                        asm volatile("" : "+v"(h4));  // the addresses below are formed here, not kept
+#pragma unroll
+                        for (int i = 0; i < 16; i++) {
+                            const int ch = 32 * d + 8 * (i >> 2) + h4 + (i & 3);
+                            const uint16_t v =
+                                *(const uint16_t *)(vt + ch * 64 + (((key >> 3) ^ ((ch >> 1) & 3)) * 16) + (key & 7) * 2);
+                            if ((v & kAttwExp<NP>) == kAttwExp<NP>) o[d][i] = __builtin_fmaf(p, attw_value<NP>(v), o[d][i]);
+                        }
+                    }
+                }
             }
         }
         const int x = bk;  // next: K in the free buffer, V in this K's, free this V's
@@ -310,7 +391,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
         __syncthreads();
     }
-    if (b == 1 || !live) return;
+    if constexpr (!CAREFUL) {
+        float nan = 0.0f;
+        if (b == 0) {
+#pragma unroll
+            for (int d = 0; d < DT; d++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) nan = __builtin_fmaf(o[d][i], 0.0f, nan);
+        }
+        if (__syncthreads_or(nan != 0.0f)) return true;  // (NaN)
+    }
+    if (b == 1 || !live) return false;
     if (a.out && t < a.M) {
         float *op = a.out + (size_t)t * a.qstride + head * D;
 #pragma unroll
@@ -346,6 +437,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             if (h == 0) pack_scale(rec, l31, blk & 7, qd, sum);
         }
     }
+    return false;
+}
+
+template <int NP, int D>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_attw(AttwArgs a) {
+    if (attw_body<NP, D, false>(a)) attw_body<NP, D, true>(a);
 }
 
 // f32 rows (FMT 0) or a Q8 cache (FMT 1) into three bfloat16 planes; slots
@@ -365,6 +462,12 @@ __global__ __launch_bounds__(256) void k_attw_split(AttwSplitArgs a) {
         }
     };
     auto put = [&](uint16_t *o, size_t at, float v) {
+        const uint32_t bits = __float_as_uint(v);
+        if ((bits & 0x7F800000u) == 0x7F800000u) {  // Inf, NaN: the first plane alone
+            o[at] = (uint16_t)(bits >> 16 | (bits & 0x007FFFFFu ? 0x40u : 0u));
+            o[a.plane + at] = o[2 * a.plane + at] = 0;
+            return;
+        }
 #pragma unroll
         for (int p = 0; p < 3; p++) {
             const uint32_t u = attw_part(__float_as_uint(v), p);

@@ -66,6 +66,80 @@ def test_values(backend, hd):
     _check(backend, 8, 2, hd, 100, edit)
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("j", [0, 40, 70, 99])
+@pytest.mark.parametrize("what", ["v nan", "v inf", "k inf", "k nan", "k large", "q inf", "all"])
+def test_not_finite(backend, hd, j, what):
+    """Values that are not finite at position j: every earlier token keeps its
+    bits, later ones get what the formula gives (an Inf score of -Inf is a key
+    of no weight, a visible Inf value an Inf), other channels and heads stay."""
+    import torch
+
+    print(f"[attw] D={hd} {what} at {j}", flush=True)
+    T, nh, nkv = 100, 6, 2
+    q = S.normal(hd, 0, T * nh * hd).reshape(T, nh, hd)
+    k = S.normal(hd, 1 << 40, T * nkv * hd).reshape(T, nkv, hd)
+    v = S.normal(hd, 2 << 40, T * nkv * hd).reshape(T, nkv, hd)
+
+    def run():
+        args = (torch.from_numpy(a.reshape(T, -1)).cuda() for a in (q, k, v))
+        return backend.prefill_attention_gpu(*args, T, nh, nkv, hd).cpu().numpy().reshape(T, nh, hd)
+
+    clean = run()
+    if what in ("v nan", "all"):
+        v[j, 0, 3] = np.nan
+    if what in ("v inf", "all"):
+        v[j, 1, [0, 9, 40]] = np.inf, -np.inf, np.nan
+    if what == "k inf":
+        k[j, 0, 5], k[j, 1, 6] = np.inf, -np.inf
+    if what in ("k nan", "all"):
+        k[j, 0, 1] = np.nan
+    if what == "k large":  # scores beyond the range of f32, of either sign
+        k[j, 0, 5], q[:, :, 5] = 3e38, np.where(np.abs(q[:, :, 5]) < 0.1, 0.1, q[:, :, 5]) * 1000
+        k[:j, :, 5], k[j + 1:, :, 5] = 0.0, 0.0
+    if what == "q inf":
+        q[j, 2, 4] = np.inf
+    got = run()
+    if what != "k large":  # (its queries differ)
+        assert np.array_equal(got[:j].view(np.uint32), clean[:j].view(np.uint32))
+    with np.errstate(all="ignore"):
+        for t in range(j, T):
+            for h in range(nh):
+                s = (k[:t + 1, h // 3] * q[t, h]).sum(1, dtype=np.float32).astype(np.float64) / np.sqrt(hd)
+                p = np.exp(s - np.fmax.reduce(s)) if not np.isposinf(s).any() else s * np.nan
+                # a key of no weight takes no part only if its value is a number
+                want = (p[:, None] * v[:t + 1, h // 3]).sum(0) / p.sum()
+                mag = (p[:, None] * np.abs(v[:t + 1, h // 3])).sum(0) / p.sum()
+                ok = np.isfinite(want)
+                assert np.array_equal(got[t, h][~ok], want[~ok].astype(np.float32), equal_nan=True), (t, h)
+                # f32 scores here and there: their error is an absolute 2^-24
+                # times ~sqrt(hd) max|score|, and the weights' relative error
+                big = np.abs(s[np.isfinite(s)]).max(initial=1.0)
+                bound = (4 * hd * big + 4 * np.sqrt(T) + 16) * 2.0 ** -24 * mag[ok]
+                assert (np.abs(got[t, h][ok] - want[ok]) <= bound).all(), (t, h)
+
+
+@pytest.mark.parametrize("kv", [FL_KV_F16, FL_KV_Q8, FL_KV_F32])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_wide_prefill_over_stale_slots(backend, kv, hd):
+    """Slots behind the prompt's last token (an earlier sequence's, rejected
+    drafts') that are not finite do not reach a wide pass, nor do rows of the
+    prompt's own other layers or tokens: the logits keep their bits."""
+    print(f"[wide] stale kv={kv} D={hd}", flush=True)
+    n = 101
+    spec = S.tiny_spec(FL_Q8_0, heads=4, kv_heads=2, head_dim=hd, hidden=512, max_seq=192)
+    backend.init_gpu_kv_cache(spec, kv)
+    backend.upload_weights_to_gpu(S.make_model(spec, seed=11))
+    toks = S.random_tokens(4, n, spec.vocab)
+    want = backend.forward_prefill(toks, 0)[0]
+    bad = np.full((64, 2 * hd), np.inf, np.float32)
+    bad[::2, ::3] = np.nan
+    for l in range(spec.layers):
+        backend.gpu_kv_write_batch(l, n, bad, bad)
+    got = backend.forward_prefill(toks, 0)[0]
+    assert np.isfinite(want).all() and np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("kv", [FL_KV_F16, FL_KV_Q8, FL_KV_F32])
 @pytest.mark.parametrize("fmt,hd,pos0,n", [(FL_Q8_0, 64, 0, 65), (FL_Q4K, 128, 37, 200), (FL_Q8_0, 128, 3, 2150)])
 def test_wide_prefill_matches_short_passes(backend, kv, fmt, hd, pos0, n):
