@@ -26,6 +26,7 @@ constexpr int kMvoThreads = 512;  // 8 waves
 constexpr int kMvoMaxTokens = 8;
 // LDS rows lie K + 8 halves apart: 16 bytes beyond a multiple of the banks, so
 // the 16 rows of an operand read (2 lane groups at a time) take every bank once
+// (LONG rows, one token: 0)
 constexpr int kMvoPad = 8;
 
 struct MvoArgs {
@@ -127,17 +128,17 @@ struct MvoUnit<F_Q8_0> {
 // pieces per wave ran the same loop 17 us slower.  KW waves per tile,
 // kMvoThreads / 64 / KW tiles per workgroup; the next unit's loads are in
 // flight while one is consumed (a third unit in flight, or 16 waves, measured
-// alike).
-template <int FMT, int KW>
+// alike).  LONG: one token whose row leaves the LDS no room for the padding and
+// both buffers of partial sums.
+template <int FMT, int KW, bool LONG>
 __global__ __launch_bounds__(kMvoThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_mvo(MvoArgs a) {
     extern __shared__ __align__(16) char smem[];
     const WDesc &W = a.W;
     const int K = W.cols, M = a.M;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kg = lane >> 4, r16 = lane & 15;
     constexpr int NW = kMvoThreads / 64, TG = NW / KW;
-    // LDS: rows m = 2t + (hi / lo) of the normed input as f16, [2*M][XS], then
-    // a row of zeros for the MFMA rows past 2M
-    const int XS = K + kMvoPad;
+    // LDS: rows m = 2t + (hi / lo) of the normed input as f16, [2*M][XS]
+    const int XS = K + (LONG ? 0 : kMvoPad);
     _Float16 *xa = (_Float16 *)smem;
     // ---- prologue, a wave per token: rmsnorm_into, split into f16 hi / lo ----
     for (int t = wave; t < M; t += NW) {
@@ -170,19 +171,18 @@ __global__ __launch_bounds__(kMvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
             *(v4h_t *)(xa + (size_t)(2 * t + 1) * XS + i) = lo;
         }
     }
-    if (2 * M < 16)
-        for (int i = threadIdx.x; i < XS / 4; i += blockDim.x)
-            *(v4h_t *)(xa + (size_t)2 * M * XS + 4 * i) = v4h_t{(_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f};
     __syncthreads();
-    // A operand row of this lane: m = r16 (token m/2, hi/lo m%2)
-    const _Float16 *xrow = xa + (size_t)min(r16, 2 * M) * XS;
+    // A operand row of this lane: m = r16 (token m/2, hi/lo m%2); past 2M the
+    // last row again, into result rows that nothing reads
+    const _Float16 *xrow = xa + (size_t)min(r16, 2 * M - 1) * XS;
     const v4fm_t zero = {0.f, 0.f, 0.f, 0.f};
 
     const int ntile = (W.rows + 15) / 16, nu = (K + 255) >> 8, upw = (nu + KW - 1) / KW;
     const int kw = wave % KW, tg = wave / KW;
     // partial sums of a tile, [2 buffers][wave][2][64]: a buffer is written
-    // again two tiles later, past the barrier between
-    __shared__ float part[2][NW][2][64];
+    // again two tiles later, past the barrier between.  LONG: [wave][16], written
+    // again after a barrier of its own.
+    __shared__ float part[LONG ? 1 : 2][NW][LONG ? 1 : 2][LONG ? 16 : 64];
     const int first = blockIdx.x * TG, step = gridDim.x * TG;
     const int niter = (ntile - first + step - 1) / step;  // the same for every wave (first < ntile)
     unsigned long long best = 0ull;
@@ -252,17 +252,23 @@ __global__ __launch_bounds__(kMvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
         if (j < upw - 1) return;
         // the tile's KW partial sums: (row, token) per thread, summed in order.
         // Only LDS is waited for: the next unit's loads stay in flight.
-        part[it & 1][wave][0][lane] = acc[0];
-        part[it & 1][wave][1][lane] = acc[1];
+        if constexpr (LONG) {
+            __syncthreads();
+            if (lane < 16) part[0][wave][0][lane] = acc[0];
+        } else {
+            part[it & 1][wave][0][lane] = acc[0];
+            part[it & 1][wave][1][lane] = acc[1];
+        }
         acc[0] = acc[1] = 0.0f;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         const int g = threadIdx.x >> 7, e = (threadIdx.x >> 6) & 1;  // tile of the group, token parity
-        if (g < TG) {
-            float v = part[it & 1][g * KW][e][lane];
+        if (LONG ? threadIdx.x < 16 : g < TG) {
+            const int buf = LONG ? 0 : it & 1;
+            float v = part[buf][g * KW][e][lane];
 #pragma unroll
-            for (int k = 1; k < KW; k++) v += part[it & 1][g * KW + k][e][lane];
+            for (int k = 1; k < KW; k++) v += part[buf][g * KW + k][e][lane];
             const int tile = first + it * step + g, n = tile * 16 + r16, t = 2 * kg + e;
             if (tile < ntile && t < M && n < W.rows) {
                 if (a.epi == EPI_STORE) a.out[(size_t)t * W.rows + n] = v;

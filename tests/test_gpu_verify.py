@@ -218,11 +218,14 @@ def test_verify_graph_replays_match_eager(backend, oracle, kv, monkeypatch):
     (FL_Q6K, 17, 256, 2), (FL_Q6K, 33, 512, 3), (FL_Q6K, 4100, 1024, 8), (FL_Q6K, 130, 2304, 7),
     (FL_Q6K, 300, 4864, 8), (FL_Q8_0, 15, 32, 5), (FL_Q8_0, 33, 96, 8), (FL_Q8_0, 513, 1056, 6),
     (FL_Q8_0, 130, 2080, 2), (FL_Q8_0, 100, 5088, 8),
+    (FL_Q6K, 40, 8704, 4), (FL_Q8_0, 40, 9216, 4), (FL_Q8_0, 70, 10176, 4), (FL_Q8_0, 40, 10176, 7),
+    (FL_Q8_0, 40, 12288, 3), (FL_Q6K, 33, 12288, 8), (FL_Q8_0, 20, 13600, 3), (FL_Q8_0, 20, 20352, 2),
+    (FL_Q8_0, 1030, 20384, 5), (FL_Q6K, 4000, 40704, 1), (FL_Q8_0, 5000, 40800, 1), (FL_Q8_0, 20, 40800, 2),
 ])
 def test_multi_token_logits_tile_edges(backend, oracle, fmt, rows, cols, M):
     """k_mvo at its edges: ragged rows, a K that gives some of the waves of a
-    tile no unit, rows that end inside one, the longest K (two launches), the
-    MFMA's zero rows (M < 8).  float64 reference; each output sums K exact
+    tile no unit, rows that end inside one, K up to the longest (a launch for
+    every few tokens, down to one), MFMA rows without a token (M < 8).  float64 reference; each output sums K exact
     products of weights and 22-bit activations: 2^-22 per product and
     (K / 16 + 16) roundings of 2^-24, all of sum |w||x|."""
     import torch
@@ -236,3 +239,20 @@ def test_multi_token_logits_tile_edges(backend, oracle, fmt, rows, cols, M):
     wd = oracle.dequant(w, fmt, rows, cols).astype(np.float64)
     bound = (2.0 ** -22 + (cols / 16 + 16) * 2.0 ** -24) * (np.abs(x) @ np.abs(wd).T)
     assert (np.abs(got - x.astype(np.float64) @ wd.T) <= bound).all()
+
+
+@pytest.mark.parametrize("hidden,M", [(9216, 4), (12288, 3), (9216, 8)])
+def test_verify_wide_hidden(backend, hidden, M):
+    """Verify of a hidden size whose rows fill the LDS: every draft's key is
+    the argmax of its row in the decode path's logits (or a value as large)."""
+    print(f"[verify] hidden={hidden} M={M}", flush=True)
+    spec = S.tiny_spec(FL_Q8_0, hidden=hidden, layers=1, vocab=300)
+    backend.init_gpu_kv_cache(spec, FL_KV_F16)
+    backend.upload_weights_to_gpu(S.make_model(spec, seed=8))
+    toks = S.random_tokens(3, M, spec.vocab)
+    rows = [backend.forward_single_token_gpu(int(t), i) for i, t in enumerate(toks)]
+    backend.reset()
+    got, vals = backend.verify(toks, 0)
+    for row, t, v in zip(rows, got, vals):
+        big = np.abs(row).max()  # 1 %: requantized activations, as everywhere here
+        assert abs(v - row[t]) <= 0.01 * big and row.max() - row[t] <= 0.01 * big
