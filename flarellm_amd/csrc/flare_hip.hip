@@ -269,6 +269,7 @@ struct fl_ctx {
     unsigned long long *d_slot = nullptr;
     char *ws = nullptr;           // workspace of the batched ops (grown to the largest call, see ws_ensure)
     size_t ws_bytes = 0;
+    size_t ws_limit = SIZE_MAX;   // FL_OPT_WORKSPACE_MIB
     // model
     bool have_cfg = false, have_weights = false;
     fl_model_config cfg{};
@@ -348,6 +349,9 @@ struct fl_ctx {
 constexpr int kVerifyMaxKsplit = 16;
 constexpr int kWideTokens = 2048;  // tokens per wide prefill pass
 constexpr size_t kWideSplitBytes = (size_t)1 << 30;  // most memory of a wide pass's f32 / Q8 key and value planes
+// operand planes of fl_op_prefill_attention at a time, if more than one kv head
+// (1531 tokens of 8 x 128 take 18 MiB, 131072 of one head 192)
+constexpr size_t kAttnWsBytes = (size_t)256 << 20;
 constexpr int kBatchRows = 2048;  // rows per GEMM of fl_op_batched_dequant_matmul (bounds its workspace)
 constexpr int kVerifyCounters = 4096;  // workgroup columns of a fused verify GEMM
 
@@ -687,10 +691,13 @@ static int ensure_part(fl_ctx *ctx, size_t floats) {
 // The batched ops' workspace: activations and partial sums of one call.  Kept
 // with the context (a hipMalloc / hipFree pair per call costs more than the
 // smaller GEMMs) and grown when a call needs more; the ops bound what a call
-// needs by walking large batches in pieces.  The ops enqueue on the context
-// stream only, so a call that follows another cannot overwrite it early; a
-// grown buffer is freed after that stream has drained.
-static int ws_ensure(fl_ctx *ctx, size_t bytes) {
+// needs by walking large batches, or kv heads, in pieces.  The ops enqueue on
+// the context stream only, so a call that follows another cannot overwrite it
+// early; a grown buffer is freed after that stream has drained.
+// spare: the caller has a form that needs less, so the context's limit applies
+// and FL_E_OOM is no error yet.
+static int ws_ensure(fl_ctx *ctx, size_t bytes, bool spare = false) {
+    if (spare && bytes > ctx->ws_limit) return fail(ctx, FL_E_OOM, "workspace of %zu bytes: over the limit", bytes);
     if (ctx->ws_bytes >= bytes) return 0;
     if (ctx->ws) {
         HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
@@ -698,7 +705,12 @@ static int ws_ensure(fl_ctx *ctx, size_t bytes) {
     }
     ctx->ws = nullptr;
     ctx->ws_bytes = 0;
-    ALLOC(ctx, ctx->ws, bytes);
+    const int rc = dev_alloc(ctx, (void **)&ctx->ws, bytes);
+    if (rc) {
+        ctx->ws = nullptr;
+        (void)hipGetLastError();  // not for the next launch to report
+        return rc;
+    }
     ctx->ws_bytes = bytes;
     return 0;
 }
@@ -762,6 +774,15 @@ int fl_set_option(fl_ctx *ctx, int option, int value) {
     case FL_OPT_VERIFY_GRAPH: ctx->verify_graph = value != 0; break;
     case FL_OPT_EXACT: ctx->exact = value != 0; break;
     case FL_OPT_FUSE_ATTN: ctx->fuse_attn = value != 0; break;
+    case FL_OPT_WORKSPACE_MIB:
+        ctx->ws_limit = value < 0 ? SIZE_MAX : (size_t)value << 20;
+        if (ctx->ws_bytes > ctx->ws_limit) {
+            HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+            (void)hipFree(ctx->ws);
+            ctx->ws = nullptr;
+            ctx->ws_bytes = 0;
+        }
+        return 0;  // (no captured pass uses it)
     default: return fail(ctx, FL_E_INVALID, "unknown option %d", option);
     }
     drop_graphs(ctx);  // captured passes bake the old choice in
@@ -2196,12 +2217,18 @@ int fl_op_batched_dequant_matmul(fl_ctx *ctx, const fl_weight *w, const float *i
     hipError_t e = hipSuccess;
     if (batch > kVerifyMaxTokens) {
         // quantize_input_q8_0_into of every row into the GEMM's packed form,
-        // then one GEMM per kBatchRows rows
-        for (int b0 = 0; b0 < batch && e == hipSuccess; b0 += kBatchRows) {
-            const int n = std::min(kBatchRows, batch - b0);
+        // then one GEMM per kBatchRows rows (fewer where the memory is not there)
+        int rows = kBatchRows;
+        for (int b0 = 0, n; b0 < batch && e == hipSuccess; b0 += n) {
+            n = std::min(rows, batch - b0);
             const BgPlan p = bgemm_plan(w->format, w->rows, cols, n, false);
             const size_t xb = pack_bytes(n, cols);
-            const int rc = ws_ensure(ctx, xb + (p.ksplit > 1 ? (size_t)p.ksplit * n * w->rows * 4 : 0));
+            const int rc = ws_ensure(ctx, xb + (p.ksplit > 1 ? (size_t)p.ksplit * n * w->rows * 4 : 0), n > kPackTile);
+            if (rc == FL_E_OOM && n > kPackTile) {
+                rows = (n / 2 + kPackTile - 1) / kPackTile * kPackTile;
+                n = 0;
+                continue;
+            }
             if (rc) return rc;
             float *o = out + (size_t)b0 * w->rows, *part = p.ksplit > 1 ? (float *)(ctx->ws + xb) : o;
             e = launch_quant_pack(ctx->stream, input + (size_t)b0 * cols, n, cols, ctx->ws);
@@ -2238,6 +2265,51 @@ int fl_op_batched_dequant_matmul(fl_ctx *ctx, const fl_weight *w, const float *i
     return 0;
 }
 
+// fl_op_prefill_attention over the rows as they are: one query per workgroup
+// row of the decode attention (24 times the time at 1531 tokens, and no
+// memory but its split partials), for when the operand planes do not fit.
+static int prefill_attention_direct(fl_ctx *ctx, const float *q, const float *k, const float *v, int seq_len,
+                                    int num_kv_heads, int G, int head_dim, float *out) {
+    // queries z0 .. z0+Z-1 per launch (grid z), each attending 0..z0+z of the
+    // token-major rows; one set of split partials and counters per query
+    const int Z = std::min(seq_len, std::max(1, 1024 / num_kv_heads));
+    int ns, chmin;
+    choose_splits(seq_len, num_kv_heads, head_dim, ns, chmin);
+    ns = std::min(ns, 8);
+    int rc = ensure_part(ctx, (size_t)Z * num_kv_heads * ns * G * (head_dim + 2));
+    if (rc) return rc;
+    const int qd = num_kv_heads * G * head_dim, n = (seq_len + Z - 1) / Z;
+    std::vector<int> starts(n);
+    for (int i = 0; i < n; i++) starts[i] = i * Z;
+    int *dstart = nullptr;
+    ALLOC(ctx, dstart, (size_t)n * 4);
+    hipError_t e = hipMemcpyAsync(dstart, starts.data(), (size_t)n * 4, hipMemcpyHostToDevice, ctx->stream);
+    for (int i = 0; e == hipSuccess && i < n; i++) {
+        AttnArgs a{};
+        a.q = q + (size_t)starts[i] * qd;
+        a.kc = k;
+        a.vc = v;
+        a.tok_stride = (long long)num_kv_heads * head_dim;  // [token][kv_head][head_dim]
+        a.head_stride = head_dim;
+        a.posp = dstart + i;
+        a.nkv = num_kv_heads;
+        a.nsplit = ns;
+        a.chmin = chmin;
+        a.single = kAttmSingle;
+        a.part = ctx->d_part;
+        a.counters = ctx->d_counters;
+        a.out = out + (size_t)starts[i] * qd;
+        a.qstride = qd;
+        a.ostride = qd;
+        e = launch_attn(FL_KV_F32, head_dim, G, ctx->stream, a, std::min(Z, seq_len - starts[i]));
+    }
+    const hipError_t es = hipStreamSynchronize(ctx->stream);
+    (void)hipFree(dstart);
+    HIPCHK(ctx, e);
+    HIPCHK(ctx, es);
+    return 0;
+}
+
 int fl_op_prefill_attention(fl_ctx *ctx, const float *q, const float *k, const float *v, int seq_len, int num_heads,
                             int num_kv_heads, int head_dim, float *out) {
     if (!ctx || !q || !k || !v || !out) return fail(ctx, FL_E_INVALID, "null argument");
@@ -2246,35 +2318,44 @@ int fl_op_prefill_attention(fl_ctx *ctx, const float *q, const float *k, const f
     const int G = num_heads / num_kv_heads;
     if (!attn_supported(head_dim, G)) return fail(ctx, FL_E_UNSUPPORTED, "head_dim %d / group %d", head_dim, G);
     // keys and values as three bfloat16 operand planes, then every query in one
-    // launch
-    const size_t slots = (size_t)(seq_len + 31) / 32 * 32, kvd = (size_t)num_kv_heads * head_dim;
-    const int rc = ws_ensure(ctx, slots * kvd * 6 * 2);
+    // launch: for all kv heads, or as many at a time as kAttnWsBytes hold
+    const size_t slots = (size_t)(seq_len + 31) / 32 * 32, head = slots * head_dim;
+    const int qd = num_heads * head_dim, kvd = num_kv_heads * head_dim;
+    int H = (int)std::min<size_t>(num_kv_heads, std::max<size_t>(1, std::min(kAttnWsBytes, ctx->ws_limit) / (12 * head)));
+    int rc = FL_E_OOM;
+    if (12 * head <= kWideSplitBytes)
+        while ((rc = ws_ensure(ctx, 12 * head * H, true)) == FL_E_OOM && H > 1) H = (H + 1) / 2;
+    if (rc == FL_E_OOM) return prefill_attention_direct(ctx, q, k, v, seq_len, num_kv_heads, G, head_dim, out);
     if (rc) return rc;
-    AttwSplitArgs s{};
-    s.k = k;
-    s.v = v;
-    s.tok_stride = (long long)kvd;  // [token][kv_head][head_dim]
-    s.head_stride = head_dim;
-    s.T = seq_len;
-    s.nkv = num_kv_heads;
-    s.plane = slots * kvd;
-    s.out_stride = slots * head_dim;
-    s.ko = (uint16_t *)ctx->ws;
-    s.vo = s.ko + 3 * s.plane;
-    AttwArgs a{};
-    a.q = q;
-    a.k = s.ko;
-    a.v = s.vo;
-    a.plane = s.plane;
-    a.head_stride = s.out_stride;
-    a.slots = (int)slots;
-    a.M = seq_len;
-    a.nkv = num_kv_heads;
-    a.group = G;
-    a.qstride = num_heads * head_dim;
-    a.out = out;
-    hipError_t e = launch_attw_split(KV_F32, head_dim, ctx->stream, s);
-    if (e == hipSuccess) e = launch_attw(3, head_dim, ctx->stream, a);
+    hipError_t e = hipSuccess;
+    for (int h0 = 0; h0 < num_kv_heads && e == hipSuccess; h0 += H) {
+        const int n = std::min(H, num_kv_heads - h0);
+        AttwSplitArgs s{};
+        s.k = k + (size_t)h0 * head_dim;
+        s.v = v + (size_t)h0 * head_dim;
+        s.tok_stride = kvd;  // [token][kv_head][head_dim]
+        s.head_stride = head_dim;
+        s.T = seq_len;
+        s.nkv = n;
+        s.plane = head * n;
+        s.out_stride = head;
+        s.ko = (uint16_t *)ctx->ws;
+        s.vo = s.ko + 3 * s.plane;
+        AttwArgs a{};
+        a.q = q + (size_t)h0 * G * head_dim;
+        a.k = s.ko;
+        a.v = s.vo;
+        a.plane = s.plane;
+        a.head_stride = head;
+        a.slots = (int)slots;
+        a.M = seq_len;
+        a.nkv = n;
+        a.group = G;
+        a.qstride = qd;
+        a.out = out + (size_t)h0 * G * head_dim;
+        e = launch_attw_split(KV_F32, head_dim, ctx->stream, s);
+        if (e == hipSuccess) e = launch_attw(3, head_dim, ctx->stream, a);
+    }
     const hipError_t es = hipStreamSynchronize(ctx->stream);
     HIPCHK(ctx, e);
     HIPCHK(ctx, es);

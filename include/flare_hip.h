@@ -134,6 +134,12 @@ const char *fl_backend_name(void);
  * MI355X (the attention role's registers halve the QKV role's occupancy), so
  * off by default. */
 #define FL_OPT_FUSE_ATTN 4
+/* FL_OPT_WORKSPACE_MIB (default -1, no limit): most MiB of workspace that a
+ * batched op (fl_op_batched_dequant_matmul of more than 32 rows,
+ * fl_op_prefill_attention) keeps with the context.  What would need more runs
+ * in smaller pieces, in the end by kernels without a workspace, as it also
+ * does where the memory cannot be had.  Frees a larger one. */
+#define FL_OPT_WORKSPACE_MIB 5
 int fl_set_option(fl_ctx *ctx, int option, int value);
 
 /* Layer probe (testing surface; no reference counterpart).  With layer >= 0,

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from flarellm_amd import FL_KV_F16, FL_KV_F32, FL_KV_Q8, FL_Q4K, FL_Q6K, FL_Q8_0
+from flarellm_amd import _lib as L
 from flarellm_amd import synth as S
 
 pytestmark = pytest.mark.gpu
@@ -64,6 +65,43 @@ def test_values(backend, hd):
         v[5] *= 1e-6
 
     _check(backend, 8, 2, hd, 100, edit)
+
+
+@pytest.fixture
+def workspace(backend):
+    """Sets the most MiB of workspace; no limit again afterwards."""
+    yield lambda mib: backend.set_option(L.FL_OPT_WORKSPACE_MIB, mib)
+    backend.set_option(L.FL_OPT_WORKSPACE_MIB, -1)
+
+
+@pytest.mark.parametrize("mib", [1, 0])
+@pytest.mark.parametrize("nh,nkv,hd,T", [(9, 3, 64, 700), (16, 8, 128, 300), (1, 1, 64, 31)])
+def test_little_workspace(backend, workspace, mib, nh, nkv, hd, T):
+    """Kv heads in pieces (1 MiB holds two or three heads here), and without a
+    workspace at all."""
+    workspace(mib)
+    _check(backend, nh, nkv, hd, T)
+
+
+def test_workspace_is_bounded(backend, workspace):
+    """375 MiB of operand planes: in two pieces (256 MiB are kept at most), the
+    same bits as in pieces of 5 heads."""
+    import torch
+
+    T, n, hd = 8000, 32, 128
+    print(f"[attw] {T} tokens of {n} kv heads", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q, k, v = (torch.randn(T, n * hd, device="cuda", generator=g) for _ in range(3))
+    torch.cuda.synchronize()
+    workspace(0)  # (frees what earlier tests left)
+    workspace(-1)
+    free = torch.cuda.mem_get_info()[0]
+    want = backend.prefill_attention_gpu(q, k, v, T, n, n, hd)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] <= (256 << 20) + want.numel() * 4 + (32 << 20)
+    workspace(64)
+    got = backend.prefill_attention_gpu(q, k, v, T, n, n, hd)
+    assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("hd", [64, 128])

@@ -73,3 +73,16 @@ def test_odd_values(backend, oracle, fmt):
         x[35, 7] = 3.0
 
     _check(backend, oracle, fmt, 160, 512, 40, edit)
+
+
+@pytest.mark.parametrize("fmt,rows,cols,batch", [(FL_Q4K, 257, 1536, 300), (FL_Q8_0, 131, 2080, 333)])
+@pytest.mark.parametrize("mib", [1, 0])
+def test_little_workspace(backend, oracle, fmt, rows, cols, batch, mib):
+    """More rows than the workspace's limit holds: fewer at a time, 32 at least."""
+    from flarellm_amd import _lib as L
+
+    backend.set_option(L.FL_OPT_WORKSPACE_MIB, mib)
+    try:
+        _check(backend, oracle, fmt, rows, cols, batch)
+    finally:
+        backend.set_option(L.FL_OPT_WORKSPACE_MIB, -1)
