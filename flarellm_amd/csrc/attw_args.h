@@ -22,6 +22,7 @@ struct AttwArgs {
     float *out;             // [M][qstride] f32, or
     char *xp;               // Q8_0 rows in packed records (bgemm_args.h) of
     int nst;                // nst steps
+    int *flag;              // host memory: set if some output is not finite; nullptr: the careful form
 };
 
 // f32 rows or cache slots -> three bfloat16 planes
@@ -34,6 +35,7 @@ struct AttwSplitArgs {
     int T, nkv;                 // slots to split, kv heads
     uint16_t *ko, *vo;          // planes out
     size_t plane, out_stride;   // elements between planes / kv heads
+    bool careful;               // for the careful form of the attention
 };
 
 }  // namespace fl

@@ -90,25 +90,23 @@ __device__ __forceinline__ float attw_other(float v) { return __shfl_xor(v, 32, 
 //
 // Values that are not finite: a masked key has p = 0, but its V row is in the
 // PV operand, and 0 * Inf is NaN; an Inf against the zero low part of p or q is
-// NaN where the product is Inf.  Every such case leaves a NaN or Inf in O, so
-// the workgroup looks at its O once, at the end (1531 queries as above: 172.2
-// us without, 170.8 with it), and if
-// one is there does its work again with CAREFUL: values of V that are not
-// finite are taken out of the operand and added for the queries that see them,
-// and scores that came out NaN are formed again in plain f32.  Every other
-// output is the same bits with and without CAREFUL.
-// Returns whether that is needed (the same for the whole workgroup).
+// NaN where the product is Inf.  Every such case leaves a NaN or Inf in O: the
+// kernel then sets *a.flag (host memory), and the caller, which waits for the
+// result in any case, does its work again with CAREFUL: values of V that are
+// not finite are taken out of the operand and added for the queries that see
+// them, and scores that came out NaN are formed again in plain f32.  Every other
+// output is the same bits with and without CAREFUL.  (Both in one kernel, the
+// second pass behind a vote of the workgroup, cost 1 to 3 us of every call: the
+// registers of the first pass's loop fell differently.)
 template <int NP, int D, bool CAREFUL>
-__device__ __forceinline__ bool attw_body(const AttwArgs &a) {
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_attw(AttwArgs a) {
     constexpr int QP = NP == 1 ? 2 : 3;  // parts of q and p
     constexpr int KS = D / 16, DT = D / 32, CH = D / 8;  // K = 16 steps, channel tiles, 16-B chunks per row
     constexpr int PLANE = 64 * D * 2, BUF = NP * PLANE;  // bytes of 64 keys
     constexpr int NL = BUF / 1024 / 8;                   // copies per wave and tile
     extern __shared__ __align__(16) char smem[];         // 3 buffers; at the end the lanes' exchange
-    int tid = threadIdx.x;
-    if constexpr (CAREFUL) asm volatile("" : "+v"(tid));  // nothing of it is kept in registers through the first pass
-    const int lane = tid & 63, l31 = lane & 31, h = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), b = wave >> 2;
+    const int lane = threadIdx.x & 63, l31 = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = wave >> 2;
     const int kvh = blockIdx.x % a.nkv;
     const int ntile = (a.M + 31) / 32, items = ntile * a.group;
     const int w = (items + 3) / 4 - 1 - blockIdx.x / a.nkv;  // longest rows first
@@ -152,8 +150,8 @@ __device__ __forceinline__ bool attw_body(const AttwArgs &a) {
     u4x_t qf[KS][QP];
     float c = (float)(1.4426950408889634 / (D == 64 ? 8.0 : 11.313708498984761));  // log2(e) * the score scale
     float qmul = 1.0f;
+    const float *qp = a.q + (size_t)min(t, a.M - 1) * a.qstride + head * D + 8 * h;
     {
-        const float *qp = a.q + (size_t)min(t, a.M - 1) * a.qstride + head * D + 8 * h;
         if constexpr (NP == 1) {
             float m = 0.0f;
 #pragma unroll
@@ -226,7 +224,7 @@ __device__ __forceinline__ bool attw_body(const AttwArgs &a) {
             }
             if constexpr (CAREFUL) {
                 // (one score at a time, indexed by selects: registers matter here, time does not)
-                const float *qp = a.q + (size_t)min(t, a.M - 1) * a.qstride + head * D;
+                const float *qr = qp - 8 * h;
                 const char *k0 = smem + bk * BUF + 32 * b * D * 2;
 #pragma unroll 1
                 for (int i = 0; i < 16; i++) {
@@ -243,7 +241,7 @@ __device__ __forceinline__ bool attw_body(const AttwArgs &a) {
                         if constexpr (NP == 3)
                             kv += attw_value<NP>(*(const uint16_t *)(kp + PLANE)) +
                                   attw_value<NP>(*(const uint16_t *)(kp + 2 * PLANE));
-                        v = __builtin_fmaf(qp[d] * qmul, kv, v);
+                        v = __builtin_fmaf(qr[d] * qmul, kv, v);
                     }
 #pragma unroll
                     for (int j = 0; j < 16; j++) s[j] = i == j ? v : s[j];
@@ -391,17 +389,7 @@ __device__ __forceinline__ bool attw_body(const AttwArgs &a) {
         }
         __syncthreads();
     }
-    if constexpr (!CAREFUL) {
-        float nan = 0.0f;
-        if (b == 0) {
-#pragma unroll
-            for (int d = 0; d < DT; d++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) nan = __builtin_fmaf(o[d][i], 0.0f, nan);
-        }
-        if (__syncthreads_or(nan != 0.0f)) return true;  // (NaN)
-    }
-    if (b == 1 || !live) return false;
+    if (b == 1 || !live) return;
     if (a.out && t < a.M) {
         float *op = a.out + (size_t)t * a.qstride + head * D;
 #pragma unroll
@@ -437,17 +425,21 @@ __device__ __forceinline__ bool attw_body(const AttwArgs &a) {
             if (h == 0) pack_scale(rec, l31, blk & 7, qd, sum);
         }
     }
-    return false;
-}
-
-template <int NP, int D>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_attw(AttwArgs a) {
-    if (attw_body<NP, D, false>(a)) attw_body<NP, D, true>(a);
+    if constexpr (!CAREFUL) {
+        float n[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int d = 0; d < DT; d++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) n[i & 3] = __builtin_fmaf(o[d][i], 0.0f, n[i & 3]);
+        if ((n[0] + n[1]) + (n[2] + n[3]) != 0.0f)  // 0 * Inf and 0 * NaN are NaN
+            __hip_atomic_store(a.flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // f32 rows (FMT 0) or a Q8 cache (FMT 1) into three bfloat16 planes; slots
-// T .. the next multiple of 32 become zeros.  grid (32-slot blocks, kv heads)
-template <int FMT, int D>
+// T .. the next multiple of 32 become zeros.  CAREFUL: Inf and NaN in the first
+// plane alone.  grid (32-slot blocks, kv heads)
+template <int FMT, int D, bool CAREFUL>
 __global__ __launch_bounds__(256) void k_attw_split(AttwSplitArgs a) {
     __shared__ float lv[32][D + 1];
     const int blk = blockIdx.x, kvh = blockIdx.y;
@@ -462,17 +454,13 @@ __global__ __launch_bounds__(256) void k_attw_split(AttwSplitArgs a) {
         }
     };
     auto put = [&](uint16_t *o, size_t at, float v) {
-        const uint32_t bits = __float_as_uint(v);
-        if ((bits & 0x7F800000u) == 0x7F800000u) {  // Inf, NaN: the first plane alone
-            o[at] = (uint16_t)(bits >> 16 | (bits & 0x007FFFFFu ? 0x40u : 0u));
-            o[a.plane + at] = o[2 * a.plane + at] = 0;
-            return;
-        }
+        if (CAREFUL && v != v) v = __uint_as_float(0x7FC00000u);
+        const bool fin = !CAREFUL || fabsf(v) < INFINITY;
 #pragma unroll
         for (int p = 0; p < 3; p++) {
             const uint32_t u = attw_part(__float_as_uint(v), p);
             o[p * a.plane + at] = (uint16_t)(u >> 16);
-            v -= __uint_as_float(u & 0xFFFF0000u);
+            v = fin ? v - __uint_as_float(u & 0xFFFF0000u) : 0.0f;
         }
     };
     const size_t base = (size_t)kvh * a.out_stride + (size_t)blk * 32 * D;

@@ -295,6 +295,7 @@ struct fl_ctx {
     float *x = nullptr, *qkv = nullptr, *attn = nullptr, *logits = nullptr;
     float *bench_out = nullptr;  // output of fl_bench_layer_kernel launches
     long long *bench_trace = nullptr;  // attention phase timestamps (FLARE_ATTN_TRACE builds)
+    int *hflag = nullptr;              // pinned: set by an attention whose output holds a value that is not finite
     char *hpin = nullptr;              // pinned host memory, in parts:
     int *hstep = nullptr;              //   (token, position) of a directly enqueued step
     char *hstage = nullptr;            //   fl_gqa_from_cache, fl_verify
@@ -749,6 +750,8 @@ int fl_ctx_create(int device, fl_ctx **out) {
     int rc = dev_alloc(c, (void **)&c->d_pos, 64);
     if (!rc) rc = dev_alloc(c, (void **)&c->d_rope_row, 2 * 512 * 4);
     if (!rc) rc = dev_alloc(c, (void **)&c->d_counters, kCounterWords * 4);
+    if (!rc && hipHostMalloc((void **)&c->hflag, 64, hipHostMallocDefault) != hipSuccess)
+        rc = fail(c, FL_E_OOM, "hipHostMalloc(64) failed");
     if (!rc) rc = dev_alloc(c, (void **)&c->d_slot, 64);
     if (rc) {
         fl_ctx_destroy(c);
@@ -846,6 +849,7 @@ void fl_ctx_destroy(fl_ctx *ctx) {
                     ctx->sskeys, ctx->ssort, ctx->ws};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    if (ctx->hflag) (void)hipHostFree(ctx->hflag);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -2328,7 +2332,7 @@ int fl_op_prefill_attention(fl_ctx *ctx, const float *q, const float *k, const f
     if (rc == FL_E_OOM) return prefill_attention_direct(ctx, q, k, v, seq_len, num_kv_heads, G, head_dim, out);
     if (rc) return rc;
     hipError_t e = hipSuccess;
-    for (int h0 = 0; h0 < num_kv_heads && e == hipSuccess; h0 += H) {
+    auto piece = [&](int h0, bool careful) {
         const int n = std::min(H, num_kv_heads - h0);
         AttwSplitArgs s{};
         s.k = k + (size_t)h0 * head_dim;
@@ -2353,12 +2357,19 @@ int fl_op_prefill_attention(fl_ctx *ctx, const float *q, const float *k, const f
         a.group = G;
         a.qstride = qd;
         a.out = out + (size_t)h0 * G * head_dim;
+        a.flag = careful ? nullptr : ctx->hflag;
+        s.careful = careful;
         e = launch_attw_split(KV_F32, head_dim, ctx->stream, s);
         if (e == hipSuccess) e = launch_attw(3, head_dim, ctx->stream, a);
+    };
+    *ctx->hflag = 0;
+    for (bool careful : {false, true}) {
+        for (int h0 = 0; h0 < num_kv_heads && e == hipSuccess; h0 += H) piece(h0, careful);
+        const hipError_t es = hipStreamSynchronize(ctx->stream);
+        HIPCHK(ctx, e);
+        HIPCHK(ctx, es);
+        if (!*(volatile int *)ctx->hflag) break;
     }
-    const hipError_t es = hipStreamSynchronize(ctx->stream);
-    HIPCHK(ctx, e);
-    HIPCHK(ctx, es);
     return 0;
 }
 
@@ -2765,7 +2776,8 @@ static bool wide_alloc(fl_ctx *ctx, int tokens) {
 
 // One wide pass of M tokens at pos0 (ids in vtok); out_mode as enqueue_verify
 // (VOUT_NONE, or the last token's key / logits, the key in vslots[0]).
-static int enqueue_wide(fl_ctx *ctx, int M, int pos0, int out_mode) {
+// careful: attention over values that are not finite
+static int enqueue_wide(fl_ctx *ctx, int M, int pos0, int out_mode, bool careful) {
     const fl_model_config &c = ctx->cfg;
     const int H = c.hidden_dim, D = c.head_dim, G = c.num_heads / c.num_kv_heads;
     const int qd = c.num_heads * D, kvd = c.num_kv_heads * D, F = c.intermediate_dim;
@@ -2819,6 +2831,7 @@ static int enqueue_wide(fl_ctx *ctx, int M, int pos0, int out_mode) {
         w.qstride = qd;
         w.xp = ap;
         w.nst = (qd + 255) / 256;
+        w.flag = careful ? nullptr : ctx->hflag;
         if (B.planes) {
             AttwSplitArgs s{};
             s.k = a.kc;
@@ -2835,6 +2848,7 @@ static int enqueue_wide(fl_ctx *ctx, int M, int pos0, int out_mode) {
             s.out_stride = B.split_plane / c.num_kv_heads;
             s.ko = (uint16_t *)(ctx->wide + B.split);
             s.vo = s.ko + 3 * s.plane;
+            s.careful = careful;
             HIPCHK(ctx, launch_attw_split(ctx->kv_format, D, st, s));
             w.k = s.ko;
             w.v = s.vo;
@@ -2894,27 +2908,37 @@ int fl_prefill(fl_ctx *ctx, const uint32_t *tokens, int n_tokens, int pos0, floa
     const int nchunks = (n_tokens + step - 1) / step;
     // host copies stay alive until the final synchronisation
     std::vector<int> tk(tokens, tokens + n_tokens), pos(nchunks);
-    int slot = 0;  // of the last token's greedy key
-    for (int k = 0; k < nchunks; k++) {
-        const int t0 = k * step, M = std::min(step, n_tokens - t0);
-        pos[k] = pos0 + t0;
-        HIPCHK(ctx, hipMemcpyAsync(ctx->vtok, tk.data() + t0, (size_t)M * 4, hipMemcpyHostToDevice, st));
-        const int mode = k + 1 < nchunks ? VOUT_NONE : out_logits ? VOUT_LAST_LOGITS : VOUT_LAST_ARGMAX;
-        if (wide && M > least) {
-            HIPCHK(ctx, hipMemcpyAsync(ctx->vpos, &pos[k], 4, hipMemcpyHostToDevice, st));
-            rc = enqueue_wide(ctx, M, pos[k], mode);
-            slot = 0;
-        } else {
-            rc = run_verify_pass(ctx, M, &pos[k], mode);
-            slot = M - 1;
+    // A wide pass whose attention met values that are not finite runs again, and
+    // what follows it, in the careful form: it writes the same slots.
+    for (bool careful : {false, true}) {
+        int slot = 0;  // of the last token's greedy key
+        *ctx->hflag = 0;
+        for (int k = 0; k < nchunks; k++) {
+            const int t0 = k * step, M = std::min(step, n_tokens - t0);
+            pos[k] = pos0 + t0;
+            HIPCHK(ctx, hipMemcpyAsync(ctx->vtok, tk.data() + t0, (size_t)M * 4, hipMemcpyHostToDevice, st));
+            const int mode = k + 1 < nchunks ? VOUT_NONE : out_logits ? VOUT_LAST_LOGITS : VOUT_LAST_ARGMAX;
+            if (wide && M > least) {
+                HIPCHK(ctx, hipMemcpyAsync(ctx->vpos, &pos[k], 4, hipMemcpyHostToDevice, st));
+                rc = enqueue_wide(ctx, M, pos[k], mode, careful);
+                slot = 0;
+            } else {
+                rc = run_verify_pass(ctx, M, &pos[k], mode);
+                slot = M - 1;
+            }
+            if (rc) return rc;
         }
-        if (rc) return rc;
+        if (out_logits) {
+            rc = read_logits(ctx, true, out_logits, out_token, out_val);
+            if (rc) return rc;
+        } else {
+            unsigned long long key = 0;
+            HIPCHK(ctx, hipMemcpyAsync(&key, ctx->vslots + slot, 8, hipMemcpyDeviceToHost, st));
+            HIPCHK(ctx, hipStreamSynchronize(st));
+            unpack_key(key, out_token, out_val);
+        }
+        if (!*(volatile int *)ctx->hflag) break;
     }
-    if (out_logits) return read_logits(ctx, true, out_logits, out_token, out_val);
-    unsigned long long key = 0;
-    HIPCHK(ctx, hipMemcpyAsync(&key, ctx->vslots + slot, 8, hipMemcpyDeviceToHost, st));
-    HIPCHK(ctx, hipStreamSynchronize(st));
-    unpack_key(key, out_token, out_val);
     return 0;
 }
 
