@@ -2709,6 +2709,16 @@ int fl_verify(fl_ctx *ctx, const uint32_t *tokens, int n_tokens, int pos0, int32
 // activations packed by the kernels that produce them) and the many-query
 // attention.  Enqueued directly: a pass is long against its launches.
 
+// The plan of a wide pass's GEMM, by its token tiles: one of 64 per shape, so
+// sizing the buffers takes at most 256 of them.  With one for every token count
+// the first prompt of a context paid 8192 searches, and so did every longer one
+// (two 8B-shaped layers: first 4096 tokens 11.95 -> 9.2 ms, 7.0 from then on;
+// prompts growing from 60 to 2000 tokens, the last 6.9 -> 3.35 ms).
+static BgPlan wide_plan(const fl_ctx *ctx, int rows, int cols, int M) {
+    return bgemm_plan(ctx->layer_fmt, rows, cols, (M + kPackTile - 1) / kPackTile * kPackTile, true);
+}
+
+// Buffers of passes of up to cap tokens (a multiple of kPackTile).
 static WideBufs wide_layout(const fl_ctx *ctx, int cap) {
     const fl_model_config &c = ctx->cfg;
     const size_t M = cap, H = c.hidden_dim, qd = (size_t)c.num_heads * c.head_dim;
@@ -2724,8 +2734,8 @@ static WideBufs wide_layout(const fl_ctx *ctx, int cap) {
     size_t part = 0;
     const size_t shapes[4][2] = {{qd + 2 * kvd, H}, {H, qd}, {2 * F, H}, {H, F}};
     for (const auto &s : shapes)
-        for (int m = 1; m <= cap; m++)
-            part = std::max(part, (size_t)bgemm_plan(ctx->layer_fmt, (int)s[0], (int)s[1], m, true).ksplit * m * s[0]);
+        for (int m = kPackTile; m <= cap; m += kPackTile)
+            part = std::max(part, (size_t)wide_plan(ctx, (int)s[0], (int)s[1], m).ksplit * m * s[0]);
     b.x = take(M * H * 4);
     b.q = take(M * qd * 4);
     b.planes = ctx->kv_format == FL_KV_F32 || ctx->kv_format == FL_KV_Q8;
@@ -2753,25 +2763,30 @@ static bool wide_possible(const fl_ctx *ctx) {
            (size_t)(c.max_seq_len + 31) / 32 * 32 * c.num_kv_heads * c.head_dim * 12 <= kWideSplitBytes;
 }
 
-// Room for passes of `tokens` tokens; false if the memory is not there (the
-// caller then runs short passes).
+// Room for passes of `tokens` tokens, or of as many as there was room for
+// before if the memory for more is not there; false if there is none (the
+// caller then runs short passes).  Grown to twice what was there at least, so a
+// conversation whose prompts get longer pays a few times and not each time.
 static bool wide_alloc(fl_ctx *ctx, int tokens) {
-    const int cap = (tokens + kPackTile - 1) / kPackTile * kPackTile;
-    if (ctx->wide_cap >= cap) return true;
+    const int old = ctx->wide_cap, need = (tokens + kPackTile - 1) / kPackTile * kPackTile;
+    if (old >= need) return true;
     if (ctx->wide) {
         if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
         (void)hipFree(ctx->wide);
     }
     ctx->wide = nullptr;
     ctx->wide_cap = 0;
-    ctx->wb = wide_layout(ctx, cap);
-    if (hipMalloc((void **)&ctx->wide, ctx->wb.total) != hipSuccess) {
+    for (int cap : {std::max(need, std::min(2 * old, kWideTokens)), need, old}) {
+        if (!cap) break;
+        ctx->wb = wide_layout(ctx, cap);
+        if (hipMalloc((void **)&ctx->wide, ctx->wb.total) == hipSuccess) {
+            ctx->wide_cap = cap;
+            return true;
+        }
         (void)hipGetLastError();
         ctx->wide = nullptr;
-        return false;
     }
-    ctx->wide_cap = cap;
-    return true;
+    return false;
 }
 
 // One wide pass of M tokens at pos0 (ids in vtok); out_mode as enqueue_verify
@@ -2792,8 +2807,9 @@ static int enqueue_wide(fl_ctx *ctx, int M, int pos0, int out_mode, bool careful
     HIPCHK(ctx, launch_v_embed(ctx->embed.format, st, ctx->embed.desc(), ctx->vtok, M, x,
                                last_logits ? logits_key(ctx) : ctx->vslots, 1));
     int ks = 0;
-    auto gemm = [&](const fl_weight &w, const char *in) {
-        const BgPlan p = bgemm_plan(w.format, w.rows, w.cols, M, true);
+    const BgPlan pqkv = wide_plan(ctx, qd + 2 * kvd, H, M), pwo = wide_plan(ctx, H, qd, M);
+    const BgPlan pgu = wide_plan(ctx, 2 * F, H, M), pdown = wide_plan(ctx, H, F, M);
+    auto gemm = [&](const fl_weight &w, const BgPlan &p, const char *in) {
         ks = p.ksplit;
         return launch_bgemm(w.format, st, w.desc(), in, M, p, part);
     };
@@ -2802,7 +2818,7 @@ static int enqueue_wide(fl_ctx *ctx, int M, int pos0, int out_mode, bool careful
         // attention block (model.rs:2016-2311); the previous layer's down
         // projection is added to x here
         HIPCHK(ctx, launch_b_resnorm(pro, st, l ? part : nullptr, ks, M, H, x, L.attn_norm, eps, xp));
-        HIPCHK(ctx, gemm(L.qkv, xp));
+        HIPCHK(ctx, gemm(L.qkv, pqkv, xp));
         AttnArgs a{};
         kv_layer_args(ctx, l, a);
         VgArgs::QkvPost qp{};
@@ -2863,12 +2879,12 @@ static int enqueue_wide(fl_ctx *ctx, int M, int pos0, int out_mode, bool careful
             w.slots = a.S;
             HIPCHK(ctx, launch_attw(1, D, st, w));
         }
-        HIPCHK(ctx, gemm(L.wo, ap));
+        HIPCHK(ctx, gemm(L.wo, pwo, ap));
         // FFN block (model.rs:2376-2543)
         HIPCHK(ctx, launch_b_resnorm(pro, st, part, ks, M, H, x, L.ffn_norm, eps, xp));
-        HIPCHK(ctx, gemm(L.gu, xp));
+        HIPCHK(ctx, gemm(L.gu, pgu, xp));
         HIPCHK(ctx, launch_b_silu(st, part, ks, M, F, hp));
-        HIPCHK(ctx, gemm(L.down, hp));
+        HIPCHK(ctx, gemm(L.down, pdown, hp));
     }
     if (out_mode == VOUT_NONE) return 0;
     // the last token's residual, then its output projection

@@ -205,6 +205,29 @@ def test_wide_prefill_matches_short_passes(backend, kv, fmt, hd, pos0, n):
         assert np.abs(a - b).max() <= 0.01 * np.abs(b).max()
 
 
+@pytest.mark.parametrize("fmt", [FL_Q8_0, FL_Q4K])
+def test_wide_prefill_buffers_grow(backend, fmt):
+    """Prompts that get longer, over buffers that grow with them (and hold more
+    than a prompt needs): the bits of a model whose first prompt it is."""
+    spec = S.tiny_spec(fmt, embed_fmt=FL_Q6K if fmt == FL_Q4K else None, output_fmt=FL_Q6K if fmt == FL_Q4K else None,
+                       hidden=512, inter=1536, max_seq=2304)
+    model = S.make_model(spec, seed=12)
+    toks = S.random_tokens(7, 2200, spec.vocab)
+    sizes = [70, 96, 97, 150, 420, 431, 1000, 2048, 2200, 333]
+    runs = []
+    for fresh in (False, True):
+        rows = []
+        for i, n in enumerate(sizes):
+            if fresh or i == 0:
+                backend.init_gpu_kv_cache(spec, FL_KV_F16)
+                backend.upload_weights_to_gpu(model)
+            print(f"[wide] grow fmt={fmt} n={n} fresh={fresh}", flush=True)
+            rows.append(backend.forward_prefill(toks[:n], 0)[0])
+        runs.append(rows)
+    for a, b in zip(*runs):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
 def test_wide_prefill_greedy_key(backend):
     """Without logits the wide pass returns the fused argmax of the same row."""
     spec = S.tiny_spec(FL_Q8_0, max_seq=256)
