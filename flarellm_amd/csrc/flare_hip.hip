@@ -586,7 +586,7 @@ static int launch_q8in(fl_ctx *ctx, const fl_weight &w, int pro, int epi, const 
 // streaming kernel keeps more bytes in flight per wave).
 static int launch_f32in(fl_ctx *ctx, const fl_weight &w, int pro, int epi, const float *x,
                         const float *nw, float eps, float *out, unsigned long long *slot, int M = 1) {
-    if ((w.format == FL_Q6K || w.format == FL_Q8_0) && (M > 1 || measure_env("FLARE_MVO_SINGLE"))) {
+    if ((w.format == FL_Q6K || w.format == FL_Q8_0) && M > 1) {
         MvoArgs a{};
         a.W = w.desc();
         a.x = x;

@@ -54,7 +54,7 @@ hipError_t launch_fmt(hipStream_t st, const MvoArgs &a) {
 }  // namespace
 
 hipError_t launch_mvo(int fmt, hipStream_t st, const MvoArgs &a) {
-    if (a.M < 1 || a.M > kMvoMaxTokens) return hipErrorInvalidValue;
+    if (a.M < 1 || a.M > kMvoMaxTokens || (a.epi != EPI_STORE && a.epi != EPI_ARGMAX)) return hipErrorInvalidValue;
     if (fmt == F_Q6K) return a.W.cols % 256 ? hipErrorInvalidValue : launch_fmt<F_Q6K>(st, a);
     if (fmt == F_Q8_0) return a.W.cols % 32 ? hipErrorInvalidValue : launch_fmt<F_Q8_0>(st, a);
     return hipErrorNotSupported;
