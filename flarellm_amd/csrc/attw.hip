@@ -11,9 +11,6 @@ hipError_t launch_one(hipStream_t st, const AttwArgs &a) {
     // three 64-key buffers, or the end's exchange of 4 x 64 x 34 floats
     constexpr size_t lds = std::max((size_t)3 * NP * 64 * D * 2, (size_t)34 * 256 * 4);
     const auto kern = k_attw<NP, D, CAREFUL>;
-    static const hipError_t attr =
-        hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (attr != hipSuccess) return attr;
     const int items = (a.M + 31) / 32 * a.group;
     hipLaunchKernelGGL(kern, dim3((unsigned)((items + 3) / 4 * a.nkv)), dim3(512), lds, st, a);
     return hipGetLastError();

@@ -10,9 +10,6 @@ template <int FMT, int TT, int NW>
 hipError_t launch_one(hipStream_t st, const BgArgs &a) {
     constexpr size_t lds = (size_t)2 * TT * kPackRec + (FMT == F_Q4K ? NW * 32 * 4 : 0);
     const auto kern = k_bgemm<FMT, TT, NW>;
-    static const hipError_t attr =
-        hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (attr != hipSuccess) return attr;
     hipLaunchKernelGGL(kern, dim3((unsigned)(a.nrt * a.ntt * a.ksplit)), dim3(NW * 64), lds, st, a);
     return hipGetLastError();
 }
