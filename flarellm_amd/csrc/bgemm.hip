@@ -14,20 +14,22 @@ hipError_t launch_one(hipStream_t st, const BgArgs &a) {
     return hipGetLastError();
 }
 
-template <int FMT, int NW>
-hipError_t launch_tt(int tt, hipStream_t st, const BgArgs &a) {
-    switch (tt) {
-    case 1: return launch_one<FMT, 1, NW>(st, a);
-    case 2: return launch_one<FMT, 2, NW>(st, a);
-    case 3: return launch_one<FMT, 3, NW>(st, a);
-    case 4: return launch_one<FMT, 4, NW>(st, a);
+template <int FMT>
+hipError_t launch_tt(int tt, int nw, hipStream_t st, const BgArgs &a) {
+    switch (10 * tt + nw) {
+    case 14: return launch_one<FMT, 1, 4>(st, a);
+    case 24: return launch_one<FMT, 2, 4>(st, a);
+    case 28: return launch_one<FMT, 2, 8>(st, a);
+    case 38: return launch_one<FMT, 3, 8>(st, a);
+    case 48: return launch_one<FMT, 4, 8>(st, a);
     }
     return hipErrorInvalidValue;
 }
 
 }  // namespace
 
-// The plan of least estimated time.  A workgroup of 8 waves, or two of 4 waves
+// The plan of least estimated time.  A workgroup of 8 waves (2 token tiles or
+// more: with one, two workgroups of 4 waves always cost less), or two of 4 waves
 // with at most 2 token tiles, fills a CU.  The costs are a least-squares fit to
 // the times of all plans of 14 shapes on MI355X (576 x 576 to 14336 x 4096 and
 // 4096 x 14336, 32 to 2048 tokens; 6 to 7 % mean error): per 256-value step,
@@ -43,13 +45,13 @@ hipError_t launch_tt(int tt, hipStream_t st, const BgArgs &a) {
 // had 2.0e-7).
 constexpr int kQ8Steps = 28;
 struct BgCost {
-    double step8[4];  // 8 waves: us per step with 1..4 token tiles
+    double step8[3];  // 8 waves: us per step with 2..4 token tiles
     double step4[2];  // 4 waves, two workgroups on a CU
     double alone[2];  // 4 waves, one on a CU
     double round, mb;
 };
-constexpr BgCost kCostQ8{{3.61, 4.27, 5.32, 6.71}, {3.34, 4.35}, {2.30, 3.21}, 2.3, 0.165};
-constexpr BgCost kCostQ4{{2.53, 3.52, 4.57, 5.81}, {2.43, 3.63}, {1.72, 2.53}, 1.6, 0.126};
+constexpr BgCost kCostQ8{{4.27, 5.32, 6.71}, {3.34, 4.35}, {2.30, 3.21}, 2.3, 0.165};
+constexpr BgCost kCostQ4{{3.52, 4.57, 5.81}, {2.43, 3.63}, {1.72, 2.53}, 1.6, 0.126};
 BgPlan bgemm_plan(int fmt, int rows, int cols, int M, bool summed) {
     const BgCost &c = fmt == F_Q8_0 ? kCostQ8 : kCostQ4;
     const double mb = (double)M * rows * 4 / 1e6;
@@ -57,7 +59,7 @@ BgPlan bgemm_plan(int fmt, int rows, int cols, int M, bool summed) {
     BgPlan best{};
     double best_us = 0;
     for (int tt = 1; tt <= std::min(4, tiles); tt++)
-        for (int nw = 8; nw >= (tt <= 2 ? 4 : 8); nw /= 2)
+        for (int nw = tt == 1 ? 4 : 8; nw >= (tt <= 2 ? 4 : 8); nw /= 2)
             for (int want = 1; want <= std::min(nst, kBgMaxSplit); want++) {
                 BgPlan p;
                 p.tt = tt;
@@ -68,7 +70,7 @@ BgPlan bgemm_plan(int fmt, int rows, int cols, int M, bool summed) {
                 p.ksplit = (nst + p.chunk - 1) / p.chunk;
                 if (p.ksplit != want || (fmt == F_Q8_0 && p.chunk > kQ8Steps)) continue;
                 const long long wgs = (long long)p.nrt * p.ntt * p.ksplit, slots = nw == 8 ? 256 : 512;
-                const double step = nw == 8 ? c.step8[tt - 1] : wgs <= 256 ? c.alone[tt - 1] : c.step4[tt - 1];
+                const double step = nw == 8 ? c.step8[tt - 2] : wgs <= 256 ? c.alone[tt - 1] : c.step4[tt - 1];
                 double us = (double)((wgs + slots - 1) / slots) * (p.chunk * step + c.round) + p.ksplit * mb * c.mb;
                 if (p.ksplit > 1) us += summed ? (p.ksplit - 1) * mb / 4 : 4.0 + p.ksplit * mb / 4;
                 if (!best.tt || us < best_us) {
@@ -96,8 +98,8 @@ hipError_t launch_bgemm(int fmt, hipStream_t st, const WDesc &W, const char *xp,
     if ((long long)p.nrt * p.nw * 32 < W.rows || (long long)p.ntt * p.tt * kPackTile < M ||
         (long long)p.ksplit * p.chunk < a.nst || (long long)(p.ksplit - 1) * p.chunk >= a.nst)
         return hipErrorInvalidValue;
-    if (fmt == F_Q4K) return p.nw == 8 ? launch_tt<F_Q4K, 8>(p.tt, st, a) : launch_tt<F_Q4K, 4>(p.tt, st, a);
-    if (fmt == F_Q8_0) return p.nw == 8 ? launch_tt<F_Q8_0, 8>(p.tt, st, a) : launch_tt<F_Q8_0, 4>(p.tt, st, a);
+    if (fmt == F_Q4K) return launch_tt<F_Q4K>(p.tt, p.nw, st, a);
+    if (fmt == F_Q8_0) return launch_tt<F_Q8_0>(p.tt, p.nw, st, a);
     return hipErrorNotSupported;
 }
 

@@ -2314,6 +2314,14 @@ static int prefill_attention_direct(fl_ctx *ctx, const float *q, const float *k,
     return 0;
 }
 
+int fl_plan_batched_matmul(int format, int rows, int cols, int batch, int summed, int *plan) {
+    if (!plan || (format != FL_Q8_0 && format != FL_Q4K) || rows < 1 || cols < 32 || batch < 1) return FL_E_INVALID;
+    const BgPlan p = bgemm_plan(format, rows, cols, batch, summed != 0);
+    const int v[6] = {p.tt, p.nw, p.nrt, p.ntt, p.ksplit, p.chunk};
+    std::copy(v, v + 6, plan);
+    return 0;
+}
+
 int fl_op_prefill_attention(fl_ctx *ctx, const float *q, const float *k, const float *v, int seq_len, int num_heads,
                             int num_kv_heads, int head_dim, float *out) {
     if (!ctx || !q || !k || !v || !out) return fail(ctx, FL_E_INVALID, "null argument");

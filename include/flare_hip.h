@@ -198,6 +198,11 @@ int fl_op_batched_matvec_q8in(fl_ctx *ctx, const fl_weight *w, int n_tokens, con
  * on the large-batch f16-MFMA GEMM, at most 2048 at once).  Synchronises. */
 int fl_op_batched_dequant_matmul(fl_ctx *ctx, const fl_weight *w, const float *input, int batch,
                                  float *out);
+/* The large-batch GEMM's tile plan for a weight of this shape and batch rows
+ * (testing surface; host only): {token tiles of 32 per workgroup, waves of 32
+ * rows per workgroup, row tiles, token tile groups, K splits, 256-value steps
+ * per split}.  summed: the result's reader sums the splits itself. */
+int fl_plan_batched_matmul(int format, int rows, int cols, int batch, int summed, int *plan);
 /* ComputeBackend::prefill_attention_gpu (model.rs:336-368; softcap 0):
  * causal attention of seq_len tokens, token t over keys / values 0..t, each
  * as cpu_grouped_query_attention (model.rs:9849-9966).  q [seq_len][nh*hd],

@@ -133,3 +133,23 @@ def test_synth_quantize_round_trip(oracle, fmt):
         assert err.max() < limit * np.abs(w).max()
         rel = np.linalg.norm(back - w) / np.linalg.norm(w)
         assert rel < {"q4k": 0.12, "q6k": 0.03}[fmt]
+
+
+def test_batched_matmul_plans():
+    """Every plan of the large-batch GEMM covers the rows, tokens and 256-value
+    steps, has a kernel, leaves no split empty and keeps Q8_0 splits short."""
+    lib = _lib().load()
+    plan = (C.c_int32 * 6)()
+    for fmt, cols in [(1, c) for c in (32, 96, 576, 2080, 8192, 14336, 65536)] + [(2, c) for c in (256, 1536, 4096, 14336)]:
+        for rows in (1, 33, 576, 2048, 14336, 128256):
+            for batch in (1, 17, 32, 33, 97, 509, 1000, 2048):
+                for summed in (0, 1):
+                    assert lib.fl_plan_batched_matmul(fmt, rows, cols, batch, summed, plan) == 0
+                    tt, nw, nrt, ntt, ks, chunk = plan
+                    steps = (cols + 255) // 256
+                    assert (tt, nw) in ((1, 4), (2, 4), (2, 8), (3, 8), (4, 8))
+                    assert nrt * nw * 32 >= rows > (nrt - 1) * nw * 32
+                    assert ntt * tt * 32 >= batch > (ntt - 1) * tt * 32
+                    assert ks * chunk >= steps > (ks - 1) * chunk and ks <= 32
+                    assert fmt == 2 or chunk <= 28
+    assert lib.fl_plan_batched_matmul(3, 64, 256, 32, 0, plan) < 0

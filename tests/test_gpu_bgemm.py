@@ -9,11 +9,14 @@ intermediate is at most twice A = sum over blocks of max|w| * sum|x|, so with
 r = K/32 + 16 roundings of relative size 2^-24 the error stays below
 2 r A 2^-24 (weights here are zero-mean normals, so a Q4_K block's offset and
 centred codes are both within twice its largest weight)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from flarellm_amd import FL_Q4K, FL_Q8_0
 from flarellm_amd import synth as S
+from flarellm_amd._lib import check
 
 pytestmark = pytest.mark.gpu
 
@@ -55,6 +58,28 @@ def test_tile_edges(backend, oracle, fmt, rows, cols, batch):
                                                  (FL_Q4K, 6145, 512, 520)])
 def test_splits_and_pieces(backend, oracle, fmt, rows, cols, batch):
     """Deep K splits, batches larger than one piece, many token groups."""
+    _check(backend, oracle, fmt, rows, cols, batch)
+
+
+# (format, token tiles, waves, K split): every kernel the planner picks from,
+# whole and split rows, at ragged sizes
+VARIANTS = [(FL_Q8_0, 1, 4, False, 102, 256, 17), (FL_Q8_0, 1, 4, True, 102, 544, 17),
+            (FL_Q8_0, 2, 4, False, 12260, 256, 65), (FL_Q8_0, 2, 4, True, 129, 800, 1134),
+            (FL_Q8_0, 2, 8, False, 13436, 256, 136), (FL_Q8_0, 2, 8, True, 133, 1344, 1347),
+            (FL_Q8_0, 3, 8, False, 9476, 256, 388), (FL_Q8_0, 3, 8, True, 131, 2368, 1712),
+            (FL_Q8_0, 4, 8, False, 11080, 256, 488), (FL_Q8_0, 4, 8, True, 133, 6176, 1253),
+            (FL_Q4K, 1, 4, False, 100, 256, 17), (FL_Q4K, 1, 4, True, 103, 1024, 17),
+            (FL_Q4K, 2, 4, False, 10844, 256, 336), (FL_Q4K, 2, 4, True, 9277, 1792, 34),
+            (FL_Q4K, 2, 8, False, 13084, 256, 132), (FL_Q4K, 2, 8, True, 129, 2304, 897),
+            (FL_Q4K, 3, 8, False, 13059, 256, 262), (FL_Q4K, 3, 8, True, 129, 3584, 1168),
+            (FL_Q4K, 4, 8, False, 13229, 256, 392), (FL_Q4K, 4, 8, True, 135, 6400, 1231)]
+
+
+@pytest.mark.parametrize("fmt,tt,nw,split,rows,cols,batch", VARIANTS)
+def test_every_variant(backend, oracle, fmt, tt, nw, split, rows, cols, batch):
+    plan = (C.c_int32 * 6)()
+    check(backend.lib.fl_plan_batched_matmul(fmt, rows, cols, batch, 0, plan), backend.ctx)
+    assert (plan[0], plan[1], plan[4] > 1) == (tt, nw, split), tuple(plan)
     _check(backend, oracle, fmt, rows, cols, batch)
 
 
