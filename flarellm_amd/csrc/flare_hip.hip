@@ -251,9 +251,8 @@ struct Layer {
 
 // The buffers of a pass of `cap` tokens, as offsets into one allocation.
 struct WideBufs {
-    size_t x, q, k, v, part, xp, ap, hp, split, total;
-    size_t split_plane;  // elements of one operand plane of K (and of V)
-    bool planes;         // f32 / Q8 caches: keys and values split per layer
+    size_t x, q, k, v, part, xp, ap, hp, total;
+    size_t split;  // operand planes of f32 / Q8 caches (one layer's at a time)
 };
 
 struct fl_ctx {
@@ -2726,6 +2725,12 @@ static BgPlan wide_plan(const fl_ctx *ctx, int rows, int cols, int M) {
     return bgemm_plan(ctx->layer_fmt, rows, cols, (M + kPackTile - 1) / kPackTile * kPackTile, true);
 }
 
+// Elements of one operand plane of an f32 / Q8 cache's keys (or values).
+static size_t split_plane_elems(const fl_ctx *ctx) {
+    const fl_model_config &c = ctx->cfg;
+    return (size_t)(c.max_seq_len + 31) / 32 * 32 * c.num_kv_heads * c.head_dim;
+}
+
 // Buffers of passes of up to cap tokens (a multiple of kPackTile).
 static WideBufs wide_layout(const fl_ctx *ctx, int cap) {
     const fl_model_config &c = ctx->cfg;
@@ -2746,7 +2751,6 @@ static WideBufs wide_layout(const fl_ctx *ctx, int cap) {
             part = std::max(part, (size_t)wide_plan(ctx, (int)s[0], (int)s[1], m).ksplit * m * s[0]);
     b.x = take(M * H * 4);
     b.q = take(M * qd * 4);
-    b.planes = ctx->kv_format == FL_KV_F32 || ctx->kv_format == FL_KV_Q8;
     const bool staged = ctx->kv_format == FL_KV_Q8;
     b.k = take(staged ? M * kvd * 4 : 0);
     b.v = take(staged ? M * kvd * 4 : 0);
@@ -2754,8 +2758,7 @@ static WideBufs wide_layout(const fl_ctx *ctx, int cap) {
     b.xp = take(pack_bytes(cap, (int)H));
     b.ap = take(pack_bytes(cap, (int)qd));
     b.hp = take(pack_bytes(cap, (int)F));
-    b.split_plane = b.planes ? (size_t)(c.max_seq_len + 31) / 32 * 32 * kvd : 0;
-    b.split = take(b.split_plane * 6 * 2);
+    b.split = take(ctx->kv_format == FL_KV_F16 ? 0 : split_plane_elems(ctx) * 6 * 2);
     b.total = at;
     return b;
 }
@@ -2768,7 +2771,7 @@ static bool wide_possible(const fl_ctx *ctx) {
     if (c.hidden_dim > kResnormMaxH) return false;
     if (ctx->kv_format == FL_KV_F16) return true;
     return (ctx->kv_format == FL_KV_F32 || ctx->kv_format == FL_KV_Q8) &&
-           (size_t)(c.max_seq_len + 31) / 32 * 32 * c.num_kv_heads * c.head_dim * 12 <= kWideSplitBytes;
+           split_plane_elems(ctx) * 12 <= kWideSplitBytes;
 }
 
 // Room for passes of `tokens` tokens, or of as many as there was room for
@@ -2797,12 +2800,86 @@ static bool wide_alloc(fl_ctx *ctx, int tokens) {
     return false;
 }
 
+// Many-query attention over one layer's cache: a has the cache, w the queries,
+// outputs and flag.  f32 and Q8 caches go through operand planes at split
+// (split_plane_elems of K, then of V, three planes each).
+static hipError_t cache_attention(fl_ctx *ctx, const AttnArgs &a, AttwArgs w, uint16_t *split) {
+    const fl_model_config &c = ctx->cfg;
+    const int D = c.head_dim;
+    w.nkv = c.num_kv_heads;
+    w.group = c.num_heads / c.num_kv_heads;
+    w.qstride = c.num_heads * D;
+    w.nst = (w.qstride + 255) / 256;
+    if (ctx->kv_format == FL_KV_F16) {
+        w.k = (const uint16_t *)a.kc;
+        w.v = (const uint16_t *)a.vc;
+        w.head_stride = a.head_stride;
+        w.slots = a.S;
+        return launch_attw(1, D, ctx->stream, w);
+    }
+    AttwSplitArgs s{};
+    s.k = a.kc;
+    s.v = a.vc;
+    s.ks = a.ks;
+    s.vs = a.vs;
+    s.tok_stride = D;
+    s.head_stride = a.head_stride;
+    s.v_tblk = a.v_tblk;
+    s.S = a.S;
+    s.T = w.pos0 + w.M;
+    s.nkv = c.num_kv_heads;
+    s.plane = split_plane_elems(ctx);
+    s.out_stride = s.plane / c.num_kv_heads;
+    s.ko = split;
+    s.vo = s.ko + 3 * s.plane;
+    s.careful = !w.flag;
+    const hipError_t e = launch_attw_split(ctx->kv_format, D, ctx->stream, s);
+    if (e != hipSuccess) return e;
+    w.k = s.ko;
+    w.v = s.vo;
+    w.plane = s.plane;
+    w.head_stride = s.out_stride;
+    w.slots = (s.T + 31) / 32 * 32;
+    return launch_attw(3, D, ctx->stream, w);
+}
+
+int fl_gqa_queries_from_cache(fl_ctx *ctx, int layer, const float *q, int n, int pos0, float *out, void *packed) {
+    if (!ctx || !q || !out) return fail(ctx, FL_E_INVALID, "null argument");
+    if (!ctx->have_cfg) return fail(ctx, FL_E_STATE, "no kv cache");
+    const fl_model_config &c = ctx->cfg;
+    if (layer < 0 || layer >= c.num_layers) return fail(ctx, FL_E_INVALID, "layer %d", layer);
+    if (n < 1 || pos0 < 0 || n > c.max_seq_len - pos0) return fail(ctx, FL_E_INVALID, "%d queries at %d", n, pos0);
+    if (!wide_possible(ctx)) return fail(ctx, FL_E_UNSUPPORTED, "kv format %d", ctx->kv_format);
+    uint16_t *split = nullptr;
+    if (ctx->kv_format != FL_KV_F16) {
+        const int rc = ws_ensure(ctx, split_plane_elems(ctx) * 6 * 2);
+        if (rc) return rc;
+        split = (uint16_t *)ctx->ws;
+    }
+    AttnArgs a{};
+    kv_layer_args(ctx, layer, a);
+    AttwArgs w{};
+    w.q = q;
+    w.M = n;
+    w.pos0 = pos0;
+    w.out = out;
+    w.xp = (char *)packed;
+    *ctx->hflag = 0;
+    for (bool careful : {false, true}) {
+        w.flag = careful ? nullptr : ctx->hflag;
+        HIPCHK(ctx, cache_attention(ctx, a, w, split));
+        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+        if (!*(volatile int *)ctx->hflag) break;
+    }
+    return 0;
+}
+
 // One wide pass of M tokens at pos0 (ids in vtok); out_mode as enqueue_verify
 // (VOUT_NONE, or the last token's key / logits, the key in vslots[0]).
 // careful: attention over values that are not finite
 static int enqueue_wide(fl_ctx *ctx, int M, int pos0, int out_mode, bool careful) {
     const fl_model_config &c = ctx->cfg;
-    const int H = c.hidden_dim, D = c.head_dim, G = c.num_heads / c.num_kv_heads;
+    const int H = c.hidden_dim, D = c.head_dim;
     const int qd = c.num_heads * D, kvd = c.num_kv_heads * D, F = c.intermediate_dim;
     const float eps = c.rms_norm_eps;
     const int pro = ctx->layer_fmt == FL_Q8_0 ? PRO_NORMQ0 : PRO_NORMQ1;
@@ -2850,43 +2927,9 @@ static int enqueue_wide(fl_ctx *ctx, int M, int pos0, int out_mode, bool careful
         w.q = qp.Q;
         w.M = M;
         w.pos0 = pos0;
-        w.nkv = c.num_kv_heads;
-        w.group = G;
-        w.qstride = qd;
         w.xp = ap;
-        w.nst = (qd + 255) / 256;
         w.flag = careful ? nullptr : ctx->hflag;
-        if (B.planes) {
-            AttwSplitArgs s{};
-            s.k = a.kc;
-            s.v = a.vc;
-            s.ks = a.ks;
-            s.vs = a.vs;
-            s.tok_stride = D;
-            s.head_stride = a.head_stride;
-            s.v_tblk = a.v_tblk;
-            s.S = a.S;
-            s.T = pos0 + M;
-            s.nkv = c.num_kv_heads;
-            s.plane = B.split_plane;
-            s.out_stride = B.split_plane / c.num_kv_heads;
-            s.ko = (uint16_t *)(ctx->wide + B.split);
-            s.vo = s.ko + 3 * s.plane;
-            s.careful = careful;
-            HIPCHK(ctx, launch_attw_split(ctx->kv_format, D, st, s));
-            w.k = s.ko;
-            w.v = s.vo;
-            w.plane = s.plane;
-            w.head_stride = s.out_stride;
-            w.slots = (s.T + 31) / 32 * 32;
-            HIPCHK(ctx, launch_attw(3, D, st, w));
-        } else {
-            w.k = (const uint16_t *)a.kc;
-            w.v = (const uint16_t *)a.vc;
-            w.head_stride = a.head_stride;
-            w.slots = a.S;
-            HIPCHK(ctx, launch_attw(1, D, st, w));
-        }
+        HIPCHK(ctx, cache_attention(ctx, a, w, (uint16_t *)(ctx->wide + B.split)));
         HIPCHK(ctx, gemm(L.wo, pwo, ap));
         // FFN block (model.rs:2376-2543)
         HIPCHK(ctx, launch_b_resnorm(pro, st, part, ks, M, H, x, L.ffn_norm, eps, xp));

@@ -297,6 +297,12 @@ int fl_kv_write_batch(fl_ctx *ctx, int layer, int pos0, int n, const float *keys
  * seq_len must be the number of tokens written (the KIVI ring holds only the
  * newest ones). */
 int fl_gqa_from_cache(fl_ctx *ctx, int layer, const float *q, int seq_len, float *out);
+/* The attention of a wide prefill pass over one layer's cache (testing
+ * surface): n queries (device, [n][nh*hd], RoPE applied), query t over slots
+ * 0 .. pos0 + t; out [n][nh*hd] f32 and, if packed is not null, the same rows
+ * as the GEMM's packed Q8_0 records (csrc/bgemm_args.h), both on the device.
+ * F32, F16 and Q8 caches.  Synchronises. */
+int fl_gqa_queries_from_cache(fl_ctx *ctx, int layer, const float *q, int n, int pos0, float *out, void *packed);
 /* Model::reset / KvCache::clear (model.rs:1591, kv_cache.rs:534-545). */
 int fl_reset(fl_ctx *ctx);
 /* forward_greedy (model.rs:1872-1942) when out_logits == NULL, else

@@ -7,6 +7,7 @@ import pytest
 from flarellm_amd import FL_KV_F16, FL_KV_F32, FL_KV_Q8, FL_Q4K, FL_Q6K, FL_Q8_0
 from flarellm_amd import _lib as L
 from flarellm_amd import synth as S
+from flarellm_amd._lib import check
 
 pytestmark = pytest.mark.gpu
 
@@ -176,6 +177,59 @@ def test_wide_prefill_over_stale_slots(backend, kv, hd):
         backend.gpu_kv_write_batch(l, n, bad, bad)
     got = backend.forward_prefill(toks, 0)[0]
     assert np.isfinite(want).all() and np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
+def _records(raw, n, cols):
+    """Packed Q8_0 records (csrc/bgemm_args.h) as codes [n][cols] and scales."""
+    rec, steps = 19456, (cols + 255) // 256
+    raw = raw.reshape((n + 31) // 32, steps, rec)
+    codes = raw[:, :, :16384].copy().view(np.float16)  # [tile][step][block][m][h][token][8]
+    codes = codes.reshape(-1, steps, 8, 2, 2, 32, 8)[..., [0, 2, 1, 3, 4, 6, 5, 7]]
+    codes = codes.transpose(0, 5, 1, 2, 4, 3, 6).reshape(-1, steps * 256)[:n, :cols]
+    scale = raw[:, :, 16384:17408].copy().view(np.float32).reshape(-1, steps, 8, 32)
+    return codes, scale.transpose(0, 3, 1, 2).reshape(-1, steps * 8)[:n, :cols // 32]
+
+
+@pytest.mark.parametrize("kv", [FL_KV_F16, FL_KV_Q8, FL_KV_F32])
+@pytest.mark.parametrize("nh,nkv,hd", [(2, 2, 64), (4, 2, 128), (9, 3, 64), (16, 4, 128), (16, 2, 64)])
+@pytest.mark.parametrize("pos0,n", [(0, 1), (0, 33), (0, 300), (5, 17), (31, 64), (64, 129), (700, 40)])
+def test_cache_attention(backend, oracle, kv, nh, nkv, hd, pos0, n):
+    """The attention of wide passes over a model's cache, every query against
+    float64 over the values that the cache holds; its packed rows hold the
+    codes of the rows it returns."""
+    import torch
+
+    print(f"[attw] cache kv={kv} heads={nh}/{nkv} D={hd} {n} at {pos0}", flush=True)
+    T, spec = pos0 + n, S.tiny_spec(FL_Q8_0, heads=nh, kv_heads=nkv, head_dim=hd, max_seq=pos0 + n + 70)
+    backend.init_gpu_kv_cache(spec, kv)
+    q = np.concatenate([np.zeros((pos0, nh * hd), np.float32), S.normal(n + hd, 0, n * nh * hd).reshape(n, -1)])
+    k, v = (S.normal(T + hd, i << 40, spec.max_seq * nkv * hd).reshape(-1, nkv * hd) for i in (1, 2))
+    v[1::7] *= 100.0
+    q[pos0 + n // 2] *= 30.0
+    backend.gpu_kv_write_batch(1, 0, k, v)  # slots behind the last query are there as well
+    k, v = k[:T], v[:T]
+    if kv != FL_KV_F32:
+        mode = oracle.OR_KV_F16 if kv == FL_KV_F16 else oracle.OR_KV_Q8
+        k, v = (a.reshape(T, -1) for a in oracle.kv_view(mode, k.reshape(T, nkv, hd), v.reshape(T, nkv, hd)))
+    got = torch.empty(n, nh * hd, device="cuda")
+    packed = torch.zeros((n + 31) // 32 * ((nh * hd + 255) // 256) * 19456, dtype=torch.uint8, device="cuda")
+    qd = torch.from_numpy(q[pos0:]).cuda()
+    torch.cuda.synchronize()
+    check(backend.lib.fl_gqa_queries_from_cache(backend.ctx, 1, qd.data_ptr(), n, pos0, got.data_ptr(),
+                                                packed.data_ptr()), backend.ctx)
+    got = got.cpu().numpy()
+    want, mag, _ = _reference(q, k, v, nh, nkv, hd)
+    sq = np.linalg.norm(q.reshape(T, nh, hd).astype(np.float64), axis=2).max() * \
+        np.linalg.norm(k.reshape(T, nkv, hd).astype(np.float64), axis=2).max() / np.sqrt(hd)
+    # the bound of _check, with 2^-22 for the two-part operands of f16 caches
+    eps = 2.0 ** (-22 if kv == FL_KV_F16 else -24)
+    bound = (4 * np.sqrt(hd) * sq + 4 * np.sqrt(T) + 16) * eps * mag[pos0:]
+    err = np.abs(got - want[pos0:])
+    assert (err <= bound + 1e-30).all(), float((err / (bound + 1e-30)).max())
+    codes, scale = _records(packed.cpu().numpy(), n, nh * hd)
+    for t in range(n):
+        c, s = oracle.quantize_q8(got[t])
+        assert np.array_equal(codes[t].astype(np.int32), c.reshape(-1)) and np.array_equal(scale[t], s.reshape(-1))
 
 
 @pytest.mark.parametrize("kv", [FL_KV_F16, FL_KV_Q8, FL_KV_F32])
