@@ -27,10 +27,9 @@ struct AttwArgs {
 
 // f32 rows or cache slots -> three bfloat16 planes
 struct AttwSplitArgs {
-    const void *k, *v;          // f32 values, or Q8 codes with ks / vs
+    const void *k, *v;          // f32 values, or Q8 codes (V in 32-slot transposed blocks) with ks / vs
     const uint16_t *ks, *vs;    // Q8: binary16 scales [kv head][S][D / 32]
     long long tok_stride, head_stride;  // elements between slots / kv heads
-    int v_tblk;                 // V in 32-slot transposed blocks (Q8 model cache)
     int S;                      // slots per kv head of the source
     int T, nkv;                 // slots to split, kv heads
     uint16_t *ko, *vo;          // planes out

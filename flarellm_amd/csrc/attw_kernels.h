@@ -448,7 +448,7 @@ __global__ __launch_bounds__(256) void k_attw_split(AttwSplitArgs a) {
         if (s >= a.T) return 0.0f;
         if constexpr (FMT == 0) {
             return ((const float *)p)[(size_t)kvh * a.head_stride + (size_t)s * a.tok_stride + d];
-        } else {
+        } else {  // V in transposed blocks [slot / 32][D][32]
             const size_t e = (size_t)kvh * a.head_stride + (tblk ? ((size_t)blk * D + d) * 32 + r : (size_t)s * D + d);
             return (float)((const int8_t *)p)[e] * h2f(sc[((size_t)kvh * a.S + s) * (D / 32) + (d >> 5)]);
         }
@@ -467,12 +467,12 @@ __global__ __launch_bounds__(256) void k_attw_split(AttwSplitArgs a) {
     for (int i = threadIdx.x; i < 32 * D; i += 256) {
         const int r = i / D, d = i % D;
         put(a.ko, base + i, value(a.k, a.ks, r, d, false));
-        if (!(FMT == 1 && a.v_tblk)) lv[r][d] = value(a.v, a.vs, r, d, false);
+        if (FMT == 0) lv[r][d] = value(a.v, a.vs, r, d, false);
     }
     __syncthreads();
     for (int i = threadIdx.x; i < 32 * D; i += 256) {
         const int d = i >> 5, r = i & 31;
-        put(a.vo, base + i, FMT == 1 && a.v_tblk ? value(a.v, a.vs, r, d, true) : lv[r][d]);
+        put(a.vo, base + i, FMT == 1 ? value(a.v, a.vs, r, d, true) : lv[r][d]);
     }
 }
 

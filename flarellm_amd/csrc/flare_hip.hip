@@ -2824,7 +2824,6 @@ static hipError_t cache_attention(fl_ctx *ctx, const AttnArgs &a, AttwArgs w, ui
     s.vs = a.vs;
     s.tok_stride = D;
     s.head_stride = a.head_stride;
-    s.v_tblk = a.v_tblk;
     s.S = a.S;
     s.T = w.pos0 + w.M;
     s.nkv = c.num_kv_heads;
