@@ -1,4 +1,6 @@
 // Many-query attention launchers (kernels in attw_kernels.h).
+#include <cmath>
+
 #include "launch.h"
 #include "attw_kernels.h"
 
@@ -6,13 +8,21 @@ namespace fl {
 
 namespace {
 
+int workgroups(int M, int nkv, int group) { return ((M + 31) / 32 * group + 3) / 4 * nkv; }
+
 template <int NP, int D, bool CAREFUL>
 hipError_t launch_one(hipStream_t st, const AttwArgs &a) {
     // three 64-key buffers, or the end's exchange of 4 x 64 x 34 floats
     constexpr size_t lds = std::max((size_t)3 * NP * 64 * D * 2, (size_t)34 * 256 * 4);
-    const auto kern = k_attw<NP, D, CAREFUL>;
-    const int items = (a.M + 31) / 32 * a.group;
-    hipLaunchKernelGGL(kern, dim3((unsigned)((items + 3) / 4 * a.nkv)), dim3(512), lds, st, a);
+    const int n = workgroups(a.M, a.nkv, a.group);
+    if (a.ksplit <= 1) {
+        hipLaunchKernelGGL((k_attw<NP, D, CAREFUL, false>), dim3((unsigned)n), dim3(512), lds, st, a);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL((k_attw<NP, D, CAREFUL, true>), dim3((unsigned)(n * a.ksplit)), dim3(512), lds, st, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_attw_merge<D>, dim3(pack_grid(a.M, (a.qstride + 1023) / 1024)), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 
@@ -31,8 +41,28 @@ hipError_t launch_split(hipStream_t st, const AttwSplitArgs &a) {
 
 }  // namespace
 
+// Splits of the keys, where the workgroups leave CUs idle (one fills a CU).  A
+// 64-key tile takes 1.3 us (D = 64) or 2.0 (D = 128) of a chain; the merge costs
+// a launch and ~0.3 us per split, so about 2 sqrt(tiles) splits, and none where
+// they would save less than that.  Measured on MI355X, 24 Q4_K layers of 1024
+// channels, 32 prompt tokens behind 500 / 8000: 1550 / 5210 us whole, 1490 /
+// 1795 split (round figures of two runs; sqrt(2 tiles) splits 1535 / 1797, tiles
+// / 4 of them 1550 / 1835), 1432 / 1825 in a short pass.
+int attw_ksplit(int M, int pos0, int nkv, int group, int &chunk) {
+    const int nit = (pos0 + M + 63) / 64;
+    const int want = std::min({kAttwSplitWgs / workgroups(M, nkv, group), (int)(2 * std::sqrt((double)nit)), kAttwMaxSplit});
+    chunk = nit * want >= 32 && want > 1 ? (nit + want - 1) / want : nit;
+    return (nit + chunk - 1) / chunk;
+}
+
+// A workgroup has 128 rows of one head, so kAttwSplitWgs of them bound this.
+size_t attw_split_floats(int D) { return (size_t)kAttwSplitWgs * 128 * (D + 2); }
+
 hipError_t launch_attw(int planes, int D, hipStream_t st, const AttwArgs &a) {
     if (a.M < 1 || a.pos0 < 0 || a.nkv < 1 || a.group < 1 || a.slots < 32 || a.slots % 32 || a.pos0 + a.M > a.slots)
+        return hipErrorInvalidValue;
+    if (a.ksplit > 1 && (!a.part || !a.ml || a.chunk < 1 || a.ksplit * workgroups(a.M, a.nkv, a.group) > kAttwSplitWgs ||
+                         (long long)a.ksplit * a.chunk * 64 < a.pos0 + a.M))
         return hipErrorInvalidValue;
     if (planes == 1) return D == 64 ? launch_form<1, 64>(st, a) : D == 128 ? launch_form<1, 128>(st, a) : hipErrorNotSupported;
     if (planes == 3) return D == 64 ? launch_form<3, 64>(st, a) : D == 128 ? launch_form<3, 128>(st, a) : hipErrorNotSupported;

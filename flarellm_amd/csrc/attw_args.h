@@ -22,6 +22,8 @@ struct AttwArgs {
     float *out;             // [M][qstride] f32, or
     char *xp;               // Q8_0 rows in packed records (bgemm_args.h) of
     int nst;                // nst steps
+    int ksplit, chunk;      // workgroups over the keys of an item, 64-key tiles of each (ksplit 0 or 1: whole)
+    float *part, *ml;       // split: [ksplit][M][qstride] f32, [ksplit][M][heads][2] (attw_split_floats)
     int *flag;              // host memory: set if some output is not finite; nullptr: the careful form
 };
 

@@ -98,7 +98,12 @@ __device__ __forceinline__ float attw_other(float v) { return __shfl_xor(v, 32, 
 // output is the same bits with and without CAREFUL.  (Both in one kernel, the
 // second pass behind a vote of the workgroup, cost 1 to 3 us of every call: the
 // registers of the first pass's loop fell differently.)
-template <int NP, int D, bool CAREFUL>
+//
+// SPLIT: few queries behind a long context have few workgroups, each a chain of
+// key tiles as long as the context.  The range of keys is then cut over
+// a.ksplit workgroups, which leave (max, sum, O) of theirs in memory for
+// k_attw_merge.  A kernel of its own: the whole form's loop is as it was.
+template <int NP, int D, bool CAREFUL, bool SPLIT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_attw(AttwArgs a) {
     constexpr int QP = NP == 1 ? 2 : 3;  // parts of q and p
     constexpr int KS = D / 16, DT = D / 32, CH = D / 8;  // K = 16 steps, channel tiles, 16-B chunks per row
@@ -109,13 +114,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = wave >> 2;
     const int kvh = blockIdx.x % a.nkv;
     const int ntile = (a.M + 31) / 32, items = ntile * a.group;
-    const int w = (items + 3) / 4 - 1 - blockIdx.x / a.nkv;  // longest rows first
+    const int nwg = (items + 3) / 4, ks = SPLIT ? blockIdx.x / a.nkv / nwg : 0;
+    const int w = nwg - 1 - (blockIdx.x / a.nkv - ks * nwg);  // longest rows first
     const int item = min(4 * w + (wave & 3), items - 1), tile = item / a.group;
     const int head = kvh * a.group + item % a.group;
     const bool live = 4 * w + (wave & 3) < items;
     // keys: the workgroup's range ends with its last query's position
     const int last_tile = (min(4 * w + 4, items) - 1) / a.group;
-    const int nkeys = a.pos0 + min(a.M, 32 * last_tile + 32), nit = (nkeys + 63) / 64;
+    const int nkeys = a.pos0 + min(a.M, 32 * last_tile + 32);
+    const int it0 = ks * a.chunk, nit = SPLIT ? min((nkeys + 63) / 64, it0 + a.chunk) : (nkeys + 63) / 64;
+    if (SPLIT && it0 >= nit) return;
     const int t = 32 * tile + l31, qpos = a.pos0 + min(t, a.M - 1);
     const int tile_last = a.pos0 + min(a.M, 32 * tile + 32) - 1;  // last key any query of this item sees
     const uint16_t *kc = a.k + (size_t)kvh * a.head_stride, *vc = a.v + (size_t)kvh * a.head_stride;
@@ -142,8 +150,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
     };
 
-    copy_k(0, smem);
-    copy_v(0, smem + BUF);
+    copy_k(SPLIT ? it0 : 0, smem);
+    copy_v(SPLIT ? it0 : 0, smem + BUF);
     // q as operands: lane = query, part p of channels 16 k + 8 h + 0..7; binary16
     // parts are scaled by a power of two per query (their residual would
     // otherwise go subnormal for small q)
@@ -187,7 +195,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const int kg = (krow & 3) | ((krow >> 1) & 4);
 
     int bk = 0, bv = 1, bn = 2;
-    for (int it = 0; it < nit; it++) {
+    for (int it = SPLIT ? it0 : 0; it < nit; it++) {
         // K of this iteration has landed (V's copies may be in flight) and
         // every wave's reads of the buffer copied to next are complete
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NL) : "memory");
@@ -375,12 +383,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if (b == 0) {
             if (d0 == 0) {
                 const float m1 = ex[32 * 256], l1 = ex[33 * 256], mn = fmaxf(m_run, m1);
-                // every query sees key 0, which is lane 0's
-                wa = __builtin_amdgcn_exp2f(m_run - mn);
+                // every query sees key 0, which is lane 0's (of split 0)
+                wa = SPLIT && m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - mn);
                 wb = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - mn);
-                const float il = 1.0f / (l_run * wa + l1 * wb);
-                wa *= il;
-                wb *= il;
+                if constexpr (SPLIT) {
+                    l_run = l_run * wa + l1 * wb;
+                    m_run = mn;
+                } else {
+                    const float il = 1.0f / (l_run * wa + l1 * wb);
+                    wa *= il;
+                    wb *= il;
+                }
             }
 #pragma unroll
             for (int d = 0; d < 2; d++)
@@ -390,14 +403,22 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         __syncthreads();
     }
     if (b == 1 || !live) return;
-    if (a.out && t < a.M) {
-        float *op = a.out + (size_t)t * a.qstride + head * D;
+    if ((SPLIT || a.out) && t < a.M) {
+        float *op = (SPLIT ? a.part + (size_t)ks * a.M * a.qstride : a.out) + (size_t)t * a.qstride + head * D;
 #pragma unroll
         for (int d = 0; d < DT; d++)
 #pragma unroll
             for (int g = 0; g < 4; g++)
                 *(v4f_t *)(op + 32 * d + 8 * g + 4 * h) =
                     v4f_t{o[d][4 * g], o[d][4 * g + 1], o[d][4 * g + 2], o[d][4 * g + 3]};
+    }
+    if constexpr (SPLIT) {
+        if (h == 0 && t < a.M) {
+            float *ml = a.ml + (((size_t)ks * a.M + t) * a.nkv * a.group + head) * 2;
+            ml[0] = m_run;
+            ml[1] = l_run;
+        }
+        return;
     }
     if (a.xp) {
         // quantize_input_q8_0_into (model.rs:5534-5571) of the row, per 32 channels
@@ -434,6 +455,39 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if ((n[0] + n[1]) + (n[2] + n[3]) != 0.0f)  // 0 * Inf and 0 * NaN are NaN
             __hip_atomic_store(a.flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
+}
+
+// The splits' (max, sum, O) into the result: 1024 channels of a token per
+// workgroup, 4 a thread (workgroups mapped as pack_wg says).
+template <int D>
+__global__ __launch_bounds__(256) void k_attw_merge(AttwArgs a) {
+    int t, chunk;
+    pack_wg((a.qstride + 1023) >> 10, t, chunk);
+    if (t >= a.M) return;
+    const int e = chunk * 1024 + 4 * threadIdx.x, ec = min(e, a.qstride - 4), nh = a.nkv * a.group;
+    // splits that hold a key which some query of the token's tile sees
+    const int last = a.pos0 + min(a.M, (t & ~31) + 32) - 1, n = min(a.ksplit, (last >> 6) / a.chunk + 1);
+    const float *ml = a.ml + ((size_t)t * nh + ec / D) * 2;
+    float m = -INFINITY, l = 0.0f;
+    for (int k = 0; k < n; k++) m = fmaxf(m, ml[(size_t)k * a.M * nh * 2]);
+    v4f_t o = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int k = 0; k < n; k++) {
+        const float mk = ml[(size_t)k * a.M * nh * 2], wk = mk == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mk - m);
+        l = __builtin_fmaf(ml[(size_t)k * a.M * nh * 2 + 1], wk, l);
+        const v4f_t p = *(const v4f_t *)(a.part + ((size_t)k * a.M + t) * a.qstride + ec);
+#pragma unroll
+        for (int j = 0; j < 4; j++) o[j] = __builtin_fmaf(p[j], wk, o[j]);
+    }
+    const float il = 1.0f / l;
+    float y[4], nan = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        y[j] = o[j] * il;
+        nan = __builtin_fmaf(y[j], 0.0f, nan);
+    }
+    if (a.flag && nan != 0.0f) __hip_atomic_store(a.flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (a.out && e < a.qstride) *(v4f_t *)(a.out + (size_t)t * a.qstride + e) = v4f_t{y[0], y[1], y[2], y[3]};
+    if (a.xp) pack_block8(y, e < a.qstride, a.xp + ((size_t)(t >> 5) * a.nst + (ec >> 8)) * kPackRec, t, e & 255);
 }
 
 // f32 rows (FMT 0) or a Q8 cache (FMT 1) into three bfloat16 planes; slots

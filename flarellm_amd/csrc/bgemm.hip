@@ -110,11 +110,6 @@ hipError_t launch_quant_pack(hipStream_t st, const float *x, int M, int K, char 
     return hipGetLastError();
 }
 
-// workgroups of kernels that map them with pack_wg: tiles in groups of 8
-static unsigned pack_grid(int M, int nchunk) {
-    return (unsigned)((M + 8 * kPackTile - 1) / (8 * kPackTile) * 8 * kPackTile * nchunk);
-}
-
 hipError_t launch_b_resnorm(int pro, hipStream_t st, const float *part, int ksplit, int M, int H, float *x,
                             const float *w, float eps, char *xp) {
     if (H % 32 || H > kResnormMaxH || M < 1) return hipErrorInvalidValue;

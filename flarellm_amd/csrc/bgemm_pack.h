@@ -40,4 +40,39 @@ __device__ __forceinline__ void pack_scale(char *rec, int t, int blk, float s, i
     }
 }
 
+// Workgroup -> (token, chunk): the 32 tokens of a tile share a record, so they
+// run on one XCD (blockIdx % 8) in a row and its L2 merges their 8-byte pieces.
+__device__ __forceinline__ void pack_wg(int nchunk, int &t, int &chunk) {
+    const int i = blockIdx.x >> 3;
+    chunk = (i >> 5) % nchunk;
+    t = (((i >> 5) / nchunk) * 8 + (blockIdx.x & 7)) * kPackTile + (i & 31);
+}
+
+// workgroups of kernels that map them with pack_wg: tiles in groups of 8
+inline unsigned pack_grid(int M, int nchunk) {
+    return (unsigned)((M + 8 * kPackTile - 1) / (8 * kPackTile) * 8 * kPackTile * nchunk);
+}
+
+// The Q8_0 block of 32 values held 4 a thread by 8 neighbouring threads, into a
+// record (quantize_input_q8_0_into arithmetic); k = the first value's index
+// within the step.
+__device__ __forceinline__ void pack_block8(const float (&y)[4], bool in, char *rec, int t, int k) {
+    float amax = fmaxf(fmaxf(fabsf(y[0]), fabsf(y[1])), fmaxf(fabsf(y[2]), fabsf(y[3])));
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+    const float d = amax / 127.0f;
+    const float id = (d != 0.0f) ? 127.0f / amax : 0.0f;
+    int q[4], sum = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        q[j] = q8_code(y[j] * id);
+        sum += q[j];
+    }
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) sum += __shfl_xor(sum, o, 64);
+    if (!in) return;
+    pack_codes4(rec, t, k, q[0], q[1], q[2], q[3]);
+    if ((k & 31) == 0) pack_scale(rec, t, k >> 5, d, sum);
+}
+
 }  // namespace fl

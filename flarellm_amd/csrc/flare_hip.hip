@@ -252,7 +252,7 @@ struct Layer {
 // The buffers of a pass of `cap` tokens, as offsets into one allocation.
 struct WideBufs {
     size_t x, q, k, v, part, xp, ap, hp, total;
-    size_t split;  // operand planes of f32 / Q8 caches (one layer's at a time)
+    size_t att;  // scratch of cache_attention (one layer's at a time)
 };
 
 struct fl_ctx {
@@ -2731,6 +2731,10 @@ static size_t split_plane_elems(const fl_ctx *ctx) {
     return (size_t)(c.max_seq_len + 31) / 32 * 32 * c.num_kv_heads * c.head_dim;
 }
 
+static size_t cache_attention_bytes(const fl_ctx *ctx) {
+    return attw_split_floats(ctx->cfg.head_dim) * 4 + (ctx->kv_format == FL_KV_F16 ? 0 : split_plane_elems(ctx) * 6 * 2);
+}
+
 // Buffers of passes of up to cap tokens (a multiple of kPackTile).
 static WideBufs wide_layout(const fl_ctx *ctx, int cap) {
     const fl_model_config &c = ctx->cfg;
@@ -2758,7 +2762,7 @@ static WideBufs wide_layout(const fl_ctx *ctx, int cap) {
     b.xp = take(pack_bytes(cap, (int)H));
     b.ap = take(pack_bytes(cap, (int)qd));
     b.hp = take(pack_bytes(cap, (int)F));
-    b.split = take(ctx->kv_format == FL_KV_F16 ? 0 : split_plane_elems(ctx) * 6 * 2);
+    b.att = take(cache_attention_bytes(ctx));
     b.total = at;
     return b;
 }
@@ -2801,15 +2805,19 @@ static bool wide_alloc(fl_ctx *ctx, int tokens) {
 }
 
 // Many-query attention over one layer's cache: a has the cache, w the queries,
-// outputs and flag.  f32 and Q8 caches go through operand planes at split
-// (split_plane_elems of K, then of V, three planes each).
-static hipError_t cache_attention(fl_ctx *ctx, const AttnArgs &a, AttwArgs w, uint16_t *split) {
+// outputs and flag; scratch (cache_attention_bytes) the partial results of a
+// split over the keys, then for f32 and Q8 caches the operand planes
+// (split_plane_elems of K, then of V, three each).
+static hipError_t cache_attention(fl_ctx *ctx, const AttnArgs &a, AttwArgs w, char *scratch) {
     const fl_model_config &c = ctx->cfg;
     const int D = c.head_dim;
     w.nkv = c.num_kv_heads;
     w.group = c.num_heads / c.num_kv_heads;
     w.qstride = c.num_heads * D;
     w.nst = (w.qstride + 255) / 256;
+    w.ksplit = attw_ksplit(w.M, w.pos0, w.nkv, w.group, w.chunk);
+    w.part = (float *)scratch;
+    w.ml = w.part + (size_t)w.ksplit * w.M * w.qstride;
     if (ctx->kv_format == FL_KV_F16) {
         w.k = (const uint16_t *)a.kc;
         w.v = (const uint16_t *)a.vc;
@@ -2829,7 +2837,7 @@ static hipError_t cache_attention(fl_ctx *ctx, const AttnArgs &a, AttwArgs w, ui
     s.nkv = c.num_kv_heads;
     s.plane = split_plane_elems(ctx);
     s.out_stride = s.plane / c.num_kv_heads;
-    s.ko = split;
+    s.ko = (uint16_t *)(scratch + attw_split_floats(D) * 4);
     s.vo = s.ko + 3 * s.plane;
     s.careful = !w.flag;
     const hipError_t e = launch_attw_split(ctx->kv_format, D, ctx->stream, s);
@@ -2849,12 +2857,8 @@ int fl_gqa_queries_from_cache(fl_ctx *ctx, int layer, const float *q, int n, int
     if (layer < 0 || layer >= c.num_layers) return fail(ctx, FL_E_INVALID, "layer %d", layer);
     if (n < 1 || pos0 < 0 || n > c.max_seq_len - pos0) return fail(ctx, FL_E_INVALID, "%d queries at %d", n, pos0);
     if (!wide_possible(ctx)) return fail(ctx, FL_E_UNSUPPORTED, "kv format %d", ctx->kv_format);
-    uint16_t *split = nullptr;
-    if (ctx->kv_format != FL_KV_F16) {
-        const int rc = ws_ensure(ctx, split_plane_elems(ctx) * 6 * 2);
-        if (rc) return rc;
-        split = (uint16_t *)ctx->ws;
-    }
+    const int rc = ws_ensure(ctx, cache_attention_bytes(ctx));
+    if (rc) return rc;
     AttnArgs a{};
     kv_layer_args(ctx, layer, a);
     AttwArgs w{};
@@ -2866,7 +2870,7 @@ int fl_gqa_queries_from_cache(fl_ctx *ctx, int layer, const float *q, int n, int
     *ctx->hflag = 0;
     for (bool careful : {false, true}) {
         w.flag = careful ? nullptr : ctx->hflag;
-        HIPCHK(ctx, cache_attention(ctx, a, w, split));
+        HIPCHK(ctx, cache_attention(ctx, a, w, ctx->ws));
         HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
         if (!*(volatile int *)ctx->hflag) break;
     }
@@ -2928,7 +2932,7 @@ static int enqueue_wide(fl_ctx *ctx, int M, int pos0, int out_mode, bool careful
         w.pos0 = pos0;
         w.xp = ap;
         w.flag = careful ? nullptr : ctx->hflag;
-        HIPCHK(ctx, cache_attention(ctx, a, w, (uint16_t *)(ctx->wide + B.split)));
+        HIPCHK(ctx, cache_attention(ctx, a, w, ctx->wide + B.att));
         HIPCHK(ctx, gemm(L.wo, pwo, ap));
         // FFN block (model.rs:2376-2543)
         HIPCHK(ctx, launch_b_resnorm(pro, st, part, ks, M, H, x, L.ffn_norm, eps, xp));

@@ -142,6 +142,9 @@ hipError_t launch_attn(int kvfmt, int D, int G, hipStream_t st, const AttnArgs &
 hipError_t launch_attq(int D, int G, hipStream_t st, const AttnArgs &a);
 // attention of many queries over one (binary16) or three (bfloat16) operand
 // planes, and the split of f32 / Q8 keys and values into the latter (attw.hip)
+constexpr int kAttwSplitWgs = 256, kAttwMaxSplit = 32;
+int attw_ksplit(int M, int pos0, int nkv, int group, int &chunk);
+size_t attw_split_floats(int D);  // partial results of any such split
 hipError_t launch_attw(int planes, int D, hipStream_t st, const AttwArgs &a);
 hipError_t launch_attw_split(int kvfmt, int D, hipStream_t st, const AttwSplitArgs &a);
 // fused QKV matvec + decode attention (fused.hip): nqwg QKV workgroups (a

@@ -158,6 +158,43 @@ def test_not_finite(backend, hd, j, what):
                 assert (np.abs(got[t, h][ok] - want[ok]) <= bound).all(), (t, h)
 
 
+@pytest.mark.parametrize("kv", [FL_KV_F16, FL_KV_F32])
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("pos0,n", [(40, 50), (2000, 40)])
+def test_cache_attention_not_finite(backend, kv, hd, pos0, n):
+    """Whole and split key ranges: a value row that is not finite is seen by the
+    queries from its position on, in its own channels and kv head; slots behind
+    the last query by none.  All else keeps its bits."""
+    import torch
+
+    print(f"[attw] cache kv={kv} D={hd} {n} at {pos0}, not finite", flush=True)
+    T, nh, nkv = pos0 + n, 4, 2
+    spec = S.tiny_spec(FL_Q8_0, heads=nh, kv_heads=nkv, head_dim=hd, max_seq=T + 70)
+    backend.init_gpu_kv_cache(spec, kv)
+    k, v = (S.normal(T, i << 40, spec.max_seq * nkv * hd).reshape(-1, nkv * hd) for i in (1, 2))
+    q = torch.from_numpy(S.normal(T, 0, n * nh * hd).reshape(n, -1)).cuda()
+
+    def run():
+        backend.gpu_kv_write_batch(0, 0, k, v)
+        out = torch.empty(n, nh * hd, device="cuda")
+        torch.cuda.synchronize()
+        check(backend.lib.fl_gqa_queries_from_cache(backend.ctx, 0, q.data_ptr(), n, pos0, out.data_ptr(), None),
+              backend.ctx)
+        return out.cpu().numpy()
+
+    clean = run()
+    j = n // 2
+    k[T:], v[T:] = np.inf, np.nan
+    v[pos0 + j, [3, 40]] = np.nan, np.inf  # kv head 0, query heads 0 and 1
+    want = clean.copy()
+    for h in (0, 1):
+        want[j:, h * hd + 3], want[j:, h * hd + 40] = np.nan, np.inf
+    got = run()
+    ok = np.isfinite(want)
+    assert np.array_equal(got[ok].view(np.uint32), clean[ok].view(np.uint32))
+    assert np.array_equal(got[~ok], want[~ok], equal_nan=True)
+
+
 @pytest.mark.parametrize("kv", [FL_KV_F16, FL_KV_Q8, FL_KV_F32])
 @pytest.mark.parametrize("hd", [64, 128])
 def test_wide_prefill_over_stale_slots(backend, kv, hd):
@@ -192,7 +229,8 @@ def _records(raw, n, cols):
 
 @pytest.mark.parametrize("kv", [FL_KV_F16, FL_KV_Q8, FL_KV_F32])
 @pytest.mark.parametrize("nh,nkv,hd", [(2, 2, 64), (4, 2, 128), (9, 3, 64), (16, 4, 128), (16, 2, 64)])
-@pytest.mark.parametrize("pos0,n", [(0, 1), (0, 33), (0, 300), (5, 17), (31, 64), (64, 129), (700, 40)])
+@pytest.mark.parametrize("pos0,n", [(0, 1), (0, 33), (0, 300), (5, 17), (31, 64), (64, 129), (700, 4), (703, 40),
+                                    (704, 64), (950, 161), (3000, 17), (5000, 97)])
 def test_cache_attention(backend, oracle, kv, nh, nkv, hd, pos0, n):
     """The attention of wide passes over a model's cache, every query against
     float64 over the values that the cache holds; its packed rows hold the
