@@ -308,7 +308,7 @@ struct fl_ctx {
     hipGraph_t graph = nullptr;
     std::map<int, hipGraphExec_t> vgraphs;  // captured verify passes, by batch size
     hipGraphExec_t gexec = nullptr;
-    hipGraphExec_t lgexec = nullptr;  // a step that returns logits (from its second call on)
+    hipGraphExec_t lgexec = nullptr;  // a step that returns logits (see kLogitsGraphAfter)
     int logit_steps = 0;
     bool graph_ready = false;
     // speculative verify buffers (allocated on first fl_verify)
@@ -1777,6 +1777,14 @@ static int capture_logits_step(fl_ctx *ctx) {
     return 0;
 }
 
+// Steps that return logits before they are captured: a context that takes a few
+// pays nothing for a graph.  Capture and instantiation cost one call 90 us (4
+// layers of 1B widths) to 350 (30 small layers, 152 launches) where the host is
+// quick, 200 to 1200 where it is slow; the replay then saves a step 4 us (1B
+// widths, 4 or 16 layers: 228 -> 224, 591 -> 588) to 35 (30 small layers, 700 ->
+// 665), on a slow host 14, 45 and 130.
+constexpr int kLogitsGraphAfter = 16;
+
 // One decode step at `pos`: the token's embedding row (embedding == nullptr)
 // or the caller's f32 embedding row.
 static int decode_step(fl_ctx *ctx, uint32_t token, const float *embedding, int pos, float *out_logits,
@@ -1797,15 +1805,11 @@ static int decode_step(fl_ctx *ctx, uint32_t token, const float *embedding, int 
         // so the pinned words are free to write.
         ctx->hstep[0] = tok;
         ctx->hstep[1] = pos;
-        // Steps with logits replay a graph from their second call on: 4 layers
-        // of 1B widths 234 -> 226 us, 2 of 8B 240 -> 236; 30 small layers (152
-        // launches) 694-713 us against 697-769, by how fast the host enqueues.
-        // Capturing on the first would make that one pay for it.
         const bool graph = use_graph() && out_logits && !embedding && ctx->probe_layer < 0 && !ctx->exact;
-        if (graph && !ctx->lgexec && ctx->logit_steps++ > 0) {
-            const int rc = capture_logits_step(ctx);
-            if (rc) return rc;
-        }
+        // (a step that cannot be captured is enqueued; no second attempt)
+        if (graph && ctx->logit_steps <= kLogitsGraphAfter && ctx->logit_steps++ == kLogitsGraphAfter &&
+            capture_logits_step(ctx))
+            (void)hipGetLastError();
         if (graph && ctx->lgexec) {
             HIPCHK(ctx, hipGraphLaunch(ctx->lgexec, ctx->stream));
         } else {
