@@ -256,7 +256,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
             // unit i and after them, so the matrix and the vector units of the
             // SIMD work at once (in the order the compiler chose, each unit's
             // MFMAs, a wait, then its multiply-adds, two 8B-shaped layers and
-            // 4096 tokens took 7.85 ms against 7.1).  What bounds it then is
+            // 4096 tokens took 7.85 ms against 6.85).  What bounds it then is
             // vector issue: ~1000 instructions and 76 MFMAs per wave and step,
             // two waves per SIMD, fill ~90 % of its slots.
             f16x_t C[TT], dd[2];

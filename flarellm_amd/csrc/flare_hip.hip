@@ -2715,10 +2715,12 @@ int fl_verify(fl_ctx *ctx, const uint32_t *tokens, int n_tokens, int pos0, int32
 }
 
 // ---- wide prefill passes --------------------------------------------------------
-// More than kPrefillTokens prompt tokens at once: the layers as in
-// enqueue_verify, with the projections on the large-batch GEMM (its
-// activations packed by the kernels that produce them) and the many-query
-// attention.  Enqueued directly: a pass is long against its launches.
+// Prompts of 17 tokens (Q4_K layers) or 65 (Q8_0) and more, up to kWideTokens at
+// once: the layers as in enqueue_verify, with the projections on the
+// large-batch GEMM (its activations packed by the kernels that produce them)
+// and the many-query attention.  Enqueued directly, 11 launches a layer: a pass
+// of narrow layers is bound by them (24 of 512 channels: 1.1 ms for 17 to 128
+// tokens), which the short pass's graph only makes up for at few tokens.
 
 // The plan of a wide pass's GEMM, by its token tiles: one of 64 per shape, so
 // sizing the buffers takes at most 256 of them.  With one for every token count
@@ -2972,10 +2974,14 @@ int fl_prefill(fl_ctx *ctx, const uint32_t *tokens, int n_tokens, int pos0, floa
     static const int C = measure_env("FLARE_PREFILL_TOKENS")
                              ? std::max(1, std::min(kPrefillTokens, atoi(measure_env("FLARE_PREFILL_TOKENS"))))
                              : kPrefillTokens;
-    // wide passes of up to kWideTokens: of Q4_K layers from 17 tokens on (two
-    // 8B-shaped layers, 64 tokens 325 us against 361 in a short pass), of Q8_0
-    // layers where one short pass does not do (1B-shaped, 64 tokens 229 against
-    // 215 us; 65 tokens 260)
+    // wide passes of up to kWideTokens: of Q4_K layers from 17 tokens on (widths
+    // of 256 to 4096, 8 to 32 layers, 24 / 32 / 64 tokens against a short pass:
+    // 4096 x 8 905 / 958 / 1171 against 1170 / 1184 / 1295 us, 2048 x 16 1130 /
+    // 1183 / 1328 against 1208 / 1232 / 1390, 512 x 24 1073 / 1091 / 1119 against
+    // 1147 / 1150 / 1194; the one that loses is 768 x 24, 1119 / 1170 / 1236
+    // against 1093 / 1100 / 1233), of Q8_0 layers where one short pass does not
+    // do (2048 x 16, 64 tokens 1430 us in a short pass, 65 tokens 1610 wide and
+    // 2340 in two short ones; 576 x 30 65 tokens 1495 and 3650)
     const int least = ctx->layer_fmt == FL_Q4K ? std::min(C, kVerifyMaxTokens) : C;
     const bool wide = n_tokens > least && wide_possible(ctx) && wide_alloc(ctx, std::min(n_tokens, kWideTokens));
     const int step = wide ? ctx->wide_cap : C;

@@ -157,9 +157,9 @@ def test_prefill_c2_shape_vs_decode_loop(backend):
 
 @pytest.mark.timeout(900)
 def test_prefill_c3_shape_vs_decode_loop(backend):
-    """C3 (Llama-3-8B Q4_K / Q6_K output, fp16 KV): a 1024-token prefill (16
-    passes of 64 tokens on the prefill GEMM, several attention splits) against
-    the prompt fed through the decode step: the last logits within the band
+    """C3 (Llama-3-8B Q4_K / Q6_K output, fp16 KV): a 1024-token prefill (one
+    wide pass: the large-batch GEMM and the many-query attention) against the
+    prompt fed through the decode step: the last logits within the band
     two valid orders of this random-weight 8B model differ by at context 1024
     (20 % of the top logit, as for verify), the greedy token equal wherever the
     top-2 gap exceeds it."""
