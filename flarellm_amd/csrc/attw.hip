@@ -43,11 +43,12 @@ hipError_t launch_split(hipStream_t st, const AttwSplitArgs &a) {
 
 // Splits of the keys, where the workgroups leave CUs idle (one fills a CU).  A
 // 64-key tile takes 1.3 us (D = 64) or 2.0 (D = 128) of a chain; the merge costs
-// a launch and ~0.3 us per split, so about 2 sqrt(tiles) splits, and none where
+// a launch and ~0.2 us per split, so about 2 sqrt(tiles) splits, and none where
 // they would save less than that.  Measured on MI355X, 24 Q4_K layers of 1024
-// channels, 32 prompt tokens behind 500 / 8000: 1550 / 5210 us whole, 1490 /
-// 1795 split (round figures of two runs; sqrt(2 tiles) splits 1535 / 1797, tiles
-// / 4 of them 1550 / 1835), 1432 / 1825 in a short pass.
+// channels, 32 prompt tokens behind 500 / 8000: 1550 / 5210 us whole, 1436 /
+// 1692 split, 1432 / 1825 in a short pass.  (With a slower merge, 1500 / 1795;
+// sqrt(2 tiles) splits 1535 / 1797, a split per 4 tiles 1550 / 1835, per 3 1520 /
+// 1885.)
 int attw_ksplit(int M, int pos0, int nkv, int group, int &chunk) {
     const int nit = (pos0 + M + 63) / 64;
     const int want = std::min({kAttwSplitWgs / workgroups(M, nkv, group), (int)(2 * std::sqrt((double)nit)), kAttwMaxSplit});

@@ -467,16 +467,38 @@ __global__ __launch_bounds__(256) void k_attw_merge(AttwArgs a) {
     const int e = chunk * 1024 + 4 * threadIdx.x, ec = min(e, a.qstride - 4), nh = a.nkv * a.group;
     // splits that hold a key which some query of the token's tile sees
     const int last = a.pos0 + min(a.M, (t & ~31) + 32) - 1, n = min(a.ksplit, (last >> 6) / a.chunk + 1);
-    const float *ml = a.ml + ((size_t)t * nh + ec / D) * 2;
+    // batches of U splits, so that their loads are in flight together (one at a
+    // time 11.5 us for 64 tokens of 16 heads x 64 and 22 splits, so 9.2)
+    constexpr int U = 8;
+    const size_t mls = (size_t)a.M * nh * 2, ps = (size_t)a.M * a.qstride;
+    const float *ml = a.ml + ((size_t)t * nh + ec / D) * 2, *part = a.part + (size_t)t * a.qstride + ec;
     float m = -INFINITY, l = 0.0f;
-    for (int k = 0; k < n; k++) m = fmaxf(m, ml[(size_t)k * a.M * nh * 2]);
-    v4f_t o = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int k = 0; k < n; k++) {
-        const float mk = ml[(size_t)k * a.M * nh * 2], wk = mk == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mk - m);
-        l = __builtin_fmaf(ml[(size_t)k * a.M * nh * 2 + 1], wk, l);
-        const v4f_t p = *(const v4f_t *)(a.part + ((size_t)k * a.M + t) * a.qstride + ec);
+    for (int k = 0; k < n; k += U) {
+        float mk[U];
 #pragma unroll
-        for (int j = 0; j < 4; j++) o[j] = __builtin_fmaf(p[j], wk, o[j]);
+        for (int u = 0; u < U; u++) mk[u] = ml[min(k + u, n - 1) * mls];
+#pragma unroll
+        for (int u = 0; u < U; u++) m = fmaxf(m, mk[u]);
+    }
+    v4f_t o = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int k = 0; k < n; k += U) {
+        float mk[U], lk[U];
+        v4f_t p[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int i = min(k + u, n - 1);
+            mk[u] = ml[i * mls];
+            lk[u] = ml[i * mls + 1];
+            p[u] = *(const v4f_t *)(part + i * ps);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (k + u >= n) break;
+            const float wk = mk[u] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mk[u] - m);
+            l = __builtin_fmaf(lk[u], wk, l);
+#pragma unroll
+            for (int j = 0; j < 4; j++) o[j] = __builtin_fmaf(p[u][j], wk, o[j]);
+        }
     }
     const float il = 1.0f / l;
     float y[4], nan = 0.0f;
