@@ -499,6 +499,10 @@ __global__ __launch_bounds__(kAttnThreads) void k_attn(AttnArgs a0) {
         for (int p = 0; p < NP; p++) {
             float vv[8];
             rows[p].getv(vv);
+            if (n < CR && tk + p * TPP >= n) {  // the last row again: 0 * Inf is NaN
+#pragma unroll
+                for (int e = 0; e < 8; e++) vv[e] = 0.0f;
+            }
 #pragma unroll
             for (int g = 0; g < G; g++) {
                 const float pr = sc[g][tk + p * TPP];

@@ -106,16 +106,18 @@ def test_workspace_is_bounded(backend, workspace):
 
 
 @pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("mib", [-1, 0])  # k_attw, the kernels without a workspace
 @pytest.mark.parametrize("j", [0, 40, 70, 99])
 @pytest.mark.parametrize("what", ["v nan", "v inf", "k inf", "k nan", "k large", "q inf", "all"])
-def test_not_finite(backend, hd, j, what):
+def test_not_finite(backend, workspace, hd, mib, j, what):
     """Values that are not finite at position j: every earlier token keeps its
     bits, later ones get what the formula gives (an Inf score of -Inf is a key
     of no weight, a visible Inf value an Inf), other channels and heads stay."""
     import torch
 
-    print(f"[attw] D={hd} {what} at {j}", flush=True)
-    T, nh, nkv = 100, 6, 2
+    print(f"[attw] D={hd} {what} at {j}, workspace {mib}", flush=True)
+    T, nh, nkv = 200, 6, 2
+    workspace(mib)
     q = S.normal(hd, 0, T * nh * hd).reshape(T, nh, hd)
     k = S.normal(hd, 1 << 40, T * nkv * hd).reshape(T, nkv, hd)
     v = S.normal(hd, 2 << 40, T * nkv * hd).reshape(T, nkv, hd)
