@@ -2273,8 +2273,8 @@ int fl_op_batched_dequant_matmul(fl_ctx *ctx, const fl_weight *w, const float *i
 }
 
 // fl_op_prefill_attention over the rows as they are: one query per workgroup
-// row of the decode attention (24 times the time at 1531 tokens, and no
-// memory but its split partials), for when the operand planes do not fit.
+// row of the decode attention, 24 times the time at 1531 tokens of 32 heads x
+// 128.  For few tokens, and for when the operand planes do not fit.
 static int prefill_attention_direct(fl_ctx *ctx, const float *q, const float *k, const float *v, int seq_len,
                                     int num_kv_heads, int G, int head_dim, float *out) {
     // queries z0 .. z0+Z-1 per launch (grid z), each attending 0..z0+z of the
@@ -2332,6 +2332,17 @@ int fl_op_prefill_attention(fl_ctx *ctx, const float *q, const float *k, const f
         return fail(ctx, FL_E_INVALID, "bad prefill attention shape");
     const int G = num_heads / num_kv_heads;
     if (!attn_supported(head_dim, G)) return fail(ctx, FL_E_UNSUPPORTED, "head_dim %d / group %d", head_dim, G);
+    // Few tokens: their attention is short against the split into planes and
+    // k_attw's prologue (28 us against 35 for 8 heads x 128 of 1 to 32 tokens).
+    // Beyond 64 the direct kernels split the keys, and their time grows with
+    // the square of the tokens: 44 us against 47 at 128 tokens of 8 heads x 128,
+    // 39 against 41 at 64 of 32 heads and 62 against 44 at 80; x 64, 34 against
+    // 35 at 110 of 4 heads (37 against 39 at 200), 41 against 34 at 80 of 16.
+    // 8 heads a group: 37 against 42 at 64 tokens of 32 x 128, 50 against 41 of
+    // 64 x 128, x 64 never ahead (33 against 29 from one token on).
+    const bool few = (long long)seq_len * seq_len * num_heads <= 1024 * head_dim;
+    if (G < 8 ? seq_len <= 64 || few : seq_len <= 64 && few && head_dim == 128)
+        return prefill_attention_direct(ctx, q, k, v, seq_len, num_kv_heads, G, head_dim, out);
     // keys and values as three bfloat16 operand planes, then every query in one
     // launch: for all kv heads, or as many at a time as kAttnWsBytes hold
     const size_t slots = (size_t)(seq_len + 31) / 32 * 32, head = slots * head_dim;

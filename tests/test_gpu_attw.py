@@ -48,7 +48,7 @@ def _check(backend, nh, nkv, hd, T, edit=None):
     assert (np.abs(got - want) <= bound + 1e-30).all(), float((np.abs(got - want) / (bound + 1e-30)).max())
 
 
-@pytest.mark.parametrize("nh,nkv,hd", [(1, 1, 64), (6, 3, 128), (9, 3, 64), (16, 4, 128), (16, 2, 64)])
+@pytest.mark.parametrize("nh,nkv,hd", [(1, 1, 64), (6, 3, 128), (9, 3, 64), (16, 4, 128), (16, 2, 64), (8, 1, 128)])
 @pytest.mark.parametrize("T", [1, 31, 32, 33, 64, 65, 97, 129, 300])
 def test_edges(backend, nh, nkv, hd, T):
     _check(backend, nh, nkv, hd, T)
