@@ -43,12 +43,38 @@ hipError_t launch_pieces(hipStream_t st, const MvoArgs &a) {
     return hipSuccess;
 }
 
-// every wave of a tile gets units: KW at most the row's 256-value units
+// Waves per tile.  The time of a workgroup is its tiles (8 / kw at once, 256
+// workgroups) times the values of its busiest wave, so a kw that leaves waves
+// without a unit in the last round, or workgroups without a tile, loses.  The
+// most waves that all get units (they read a row in one piece), unless another
+// kw takes a tenth off.  Measured on MI355X, call time of 2 tokens with 8 (6
+// units and less: 4, 3 and less: 2) waves against the kw taken: 64000 x 2304
+// Q8_0 104.8 -> 84.0 us (1 wave), 100000 x 2304 Q6_K 104.6 -> 97.1 (2), 64000 x
+// 3072 Q8_0 133.4 -> 114.2 (4), 64000 x 1536 Q8_0 88.8 -> 79.7 (2), 20000 x 576
+// Q8_0 49.7 -> 47.8 (1), 8000 x 576 46.0 -> 44.8 (4).
+int mvo_waves(int rows, int K) {
+    const int tiles = (rows + 15) / 16, nu = (K + 255) / 256;
+    if (mvo_lds(1, K) > kMvoDynLds) return 8;  // LONG
+    auto cost = [&](int kw) {
+        const int upw = (nu + kw - 1) / kw, slots = 256 * (8 / kw);
+        const int values = (nu - 1) % kw ? upw * 256 : K - (nu - upw) * 256;  // of wave 0
+        return (long long)((tiles + slots - 1) / slots) * values;
+    };
+    const int most = nu >= 8 ? 8 : nu >= 4 ? 4 : 2;
+    int best = most;
+    for (int kw : {8, 4, 2, 1})
+        if (10 * cost(kw) <= 9 * cost(most) && cost(kw) < cost(best)) best = kw;
+    return best;
+}
+
 template <int FMT>
 hipError_t launch_fmt(hipStream_t st, const MvoArgs &a) {
-    const int nu = (a.W.cols + 255) / 256;
-    if (nu >= 8) return launch_pieces<FMT, 8>(st, a);
-    return nu >= 4 ? launch_pieces<FMT, 4>(st, a) : launch_pieces<FMT, 2>(st, a);
+    switch (mvo_waves(a.W.rows, a.W.cols)) {
+    case 8: return launch_pieces<FMT, 8>(st, a);
+    case 4: return launch_pieces<FMT, 4>(st, a);
+    case 2: return launch_pieces<FMT, 2>(st, a);
+    }
+    return launch_pieces<FMT, 1>(st, a);
 }
 
 }  // namespace

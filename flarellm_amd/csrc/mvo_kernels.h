@@ -125,7 +125,7 @@ struct MvoUnit<F_Q8_0> {
 // 245 us with 4-byte loads, a branch around every activation read and a wave
 // per tile).  The waves of a workgroup share a tile and split its K, unit by
 // unit, so together they read KiBs of each row in a row: 16 rows in 256-byte
-// pieces per wave ran the same loop 17 us slower.  KW waves per tile,
+// pieces per wave ran the same loop 17 us slower.  KW waves per tile (mvo_waves),
 // kMvoThreads / 64 / KW tiles per workgroup; the next unit's loads are in
 // flight while one is consumed (a third unit in flight, or 16 waves, measured
 // alike).  LONG: one token whose row leaves the LDS no room for the padding and
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(kMvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
     __shared__ float part[LONG ? 1 : 2][NW][LONG ? 1 : 2][LONG ? 16 : 64];
     const int first = blockIdx.x * TG, step = gridDim.x * TG;
     const int niter = (ntile - first + step - 1) / step;  // the same for every wave (first < ntile)
-    unsigned long long best = 0ull;
+    unsigned long long best[2] = {0ull, 0ull};  // KW 1: tokens 2kg, 2kg+1; else one
     float acc[2] = {0.0f, 0.0f};  // tokens 2kg, 2kg+1
     MvoUnit<FMT> ta, tb;
     auto load = [&](MvoUnit<FMT> &T, int f) {
@@ -250,6 +250,18 @@ __global__ __launch_bounds__(kMvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
             }
         }
         if (j < upw - 1) return;
+        if constexpr (KW == 1) {  // a wave's own tile
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const int tile = first + it * step + tg, n = tile * 16 + r16, t = 2 * kg + e;
+                if (tile < ntile && t < M && n < W.rows) {
+                    if (a.epi == EPI_STORE) a.out[(size_t)t * W.rows + n] = acc[e];
+                    else best[e] = umax64(best[e], argmax_key(acc[e], (uint32_t)n));
+                }
+                acc[e] = 0.0f;
+            }
+            return;
+        }
         // the tile's KW partial sums: (row, token) per thread, summed in order.
         // Only LDS is waited for: the next unit's loads stay in flight.
         if constexpr (LONG) {
@@ -272,7 +284,7 @@ __global__ __launch_bounds__(kMvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
             const int tile = first + it * step + g, n = tile * 16 + r16, t = 2 * kg + e;
             if (tile < ntile && t < M && n < W.rows) {
                 if (a.epi == EPI_STORE) a.out[(size_t)t * W.rows + n] = v;
-                else best = umax64(best, argmax_key(v, (uint32_t)n));
+                else best[0] = umax64(best[0], argmax_key(v, (uint32_t)n));
             }
         }
     };
@@ -283,9 +295,12 @@ __global__ __launch_bounds__(kMvoThreads) __attribute__((amdgpu_waves_per_eu(2, 
         // workgroup's tiles, then one device atomic per token
         __shared__ unsigned long long lb[TG][kMvoMaxTokens];
 #pragma unroll
-        for (int o = 1; o < 16; o <<= 1) best = umax64(best, __shfl_xor(best, o, 64));
-        const int g = threadIdx.x >> 7, t = 2 * kg + ((threadIdx.x >> 6) & 1);
-        if (g < TG && r16 == 0) lb[g][t] = best;
+        for (int e = 0; e < (KW == 1 ? 2 : 1); e++) {
+#pragma unroll
+            for (int o = 1; o < 16; o <<= 1) best[e] = umax64(best[e], __shfl_xor(best[e], o, 64));
+            const int g = KW == 1 ? wave : threadIdx.x >> 7, t = 2 * kg + (KW == 1 ? e : (threadIdx.x >> 6) & 1);
+            if (g < TG && r16 == 0) lb[g][t] = best[e];
+        }
         __syncthreads();
         if (threadIdx.x < M) {
             unsigned long long b = lb[0][threadIdx.x];

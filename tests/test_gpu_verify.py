@@ -221,11 +221,13 @@ def test_verify_graph_replays_match_eager(backend, oracle, kv, monkeypatch):
     (FL_Q6K, 40, 8704, 4), (FL_Q8_0, 40, 9216, 4), (FL_Q8_0, 70, 10176, 4), (FL_Q8_0, 40, 10176, 7),
     (FL_Q8_0, 40, 12288, 3), (FL_Q6K, 33, 12288, 8), (FL_Q8_0, 20, 13600, 3), (FL_Q8_0, 20, 20352, 2),
     (FL_Q8_0, 1030, 20384, 5), (FL_Q6K, 4000, 40704, 1), (FL_Q8_0, 5000, 40800, 1), (FL_Q8_0, 20, 40800, 2),
+    (FL_Q8_0, 20001, 576, 7), (FL_Q8_0, 33000, 96, 3), (FL_Q6K, 20003, 256, 8), (FL_Q6K, 9001, 1792, 5), (FL_Q8_0, 5000, 576, 8),
 ])
 def test_multi_token_logits_tile_edges(backend, oracle, fmt, rows, cols, M):
     """k_mvo at its edges: ragged rows, a K that gives some of the waves of a
     tile no unit, rows that end inside one, K up to the longest (a launch for
-    every few tokens, down to one), MFMA rows without a token (M < 8).  float64 reference; each output sums K exact
+    every few tokens, down to one), MFMA rows without a token (M < 8), 1 to 8
+    waves a tile.  float64 reference; each output sums K exact
     products of weights and 22-bit activations: 2^-22 per product and
     (K / 16 + 16) roundings of 2^-24, all of sum |w||x|."""
     import torch
@@ -241,12 +243,13 @@ def test_multi_token_logits_tile_edges(backend, oracle, fmt, rows, cols, M):
     assert (np.abs(got - x.astype(np.float64) @ wd.T) <= bound).all()
 
 
-@pytest.mark.parametrize("hidden,M", [(9216, 4), (12288, 3), (9216, 8)])
-def test_verify_wide_hidden(backend, hidden, M):
-    """Verify of a hidden size whose rows fill the LDS: every draft's key is
-    the argmax of its row in the decode path's logits (or a value as large)."""
+@pytest.mark.parametrize("hidden,M,vocab", [(9216, 4, 300), (12288, 3, 300), (9216, 8, 300), (576, 5, 20003)])
+def test_verify_wide_hidden(backend, hidden, M, vocab):
+    """Verify of a hidden size whose rows fill the LDS, and of one whose output
+    projection has a tile to every wave: every draft's key is the argmax of its
+    row in the decode path's logits (or a value as large)."""
     print(f"[verify] hidden={hidden} M={M}", flush=True)
-    spec = S.tiny_spec(FL_Q8_0, hidden=hidden, layers=1, vocab=300)
+    spec = S.tiny_spec(FL_Q8_0, hidden=hidden, layers=1, vocab=vocab)
     backend.init_gpu_kv_cache(spec, FL_KV_F16)
     backend.upload_weights_to_gpu(S.make_model(spec, seed=8))
     toks = S.random_tokens(3, M, spec.vocab)
