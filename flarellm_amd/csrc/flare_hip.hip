@@ -1783,7 +1783,7 @@ static int capture_logits_step(fl_ctx *ctx) {
 // quick, 200 to 1200 where it is slow; the replay then saves a step 4 us (1B
 // widths, 4 or 16 layers: 228 -> 224, 591 -> 588) to 35 (30 small layers, 700 ->
 // 665), on a slow host 14, 45 and 130.
-constexpr int kLogitsGraphAfter = 16;
+constexpr int kLogitsGraphAfter = 8;
 
 // One decode step at `pos`: the token's embedding row (embedding == nullptr)
 // or the caller's f32 embedding row.

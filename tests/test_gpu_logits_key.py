@@ -69,7 +69,7 @@ def test_key_skips_what_is_not_a_number(backend):
 
 
 def test_replayed_logits_steps_match_the_first(backend):
-    """Steps with logits replay a graph after the first 16: every one of 40
+    """Steps with logits replay a graph after the first 8: every one of 40
     against the same step enqueued directly (FL_OPT_EXACT off and on drops the
     graph), with other work and synchronizations between."""
     from flarellm_amd import _lib as L
